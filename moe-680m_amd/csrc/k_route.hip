@@ -78,6 +78,7 @@ hipError_t launch_router_topk(const float *logits, int M, int E, int renorm, uin
 // at M = 1 with an agent-scope release / acquire pair (each writes back / invalidates the XCD's
 // whole L2), 6.2 us with write-through stores and system-scope loads instead, against 5.6 us.
 constexpr int RG_WAVES = 4; // experts per workgroup
+constexpr int RG_GEMV_MAX_WAVES = 1024; // waves of the 4-token form (4 per CU); beyond: k_router_gemm
 
 struct RouterGemvArgs {
     const void *wg;
@@ -164,18 +165,226 @@ __global__ __launch_bounds__(64 * RG_WAVES) void k_router_gemv(RouterGemvArgs a)
     }
 }
 
+// ---------------------------------------------------------------- router gate product, many tokens
+// The same logits as a matrix product on the f32 matrix cores (v_mfma_f32_16x16x4_f32: f32
+// operands and sums, the weights exact in f32, so again only f32 rounding).  A workgroup owns
+// TILE x TILE logits (tokens x experts) and its NW waves split K, each keeping its partial block
+// in registers; x and Wg go straight from memory into MFMA operands, a ring of ND 32-K stages in
+// flight (no LDS: the waves share no operand), the partial blocks are summed through LDS, and the
+// tokens' RMSNorm factors come from the same x registers.
+// K inside a stage: the order is free as long as both operands agree.  Lane (g, i) takes K =
+// 16 q + 4 g + j of row i (q < 2, j < 4), so the four lanes of a row read 64 consecutive bytes of
+// x per load (with 32 consecutive K per lane pair the loads, one cache line per lane, took as long
+// as the MFMAs), and one IQ4_XS qs dword has the lane's 8 weights: low nibbles q = 0, high q = 1.
+// Rounding: an MFMA chain covers one stage (32 K); the chains are added in f32 per wave and the
+// waves' sums and the RMSNorm factor taken in f64.  Relative 2-norm against f64 (E = 256): 1.2e-7
+// (1.34e-7 in the 64 x 64 form) for every gate type, the one-row form 1.34e-7 (IQ4_XS 2.6e-7).
+// f16 gate, M = 4096: 947 -> 48 us; the f32 matrix cores alone need 31 us at their measured
+// 139 TFLOP/s.
+template <int WT>
+struct RmW; // a lane's 8 weights of one stage as loaded; off: byte offset of the lane's first one
+template <>
+struct RmW<MOE_WG_F32> {
+    f32x4 v[2];
+    static __device__ __forceinline__ uint32_t offset(int H, int e, int g) { return ((uint32_t)e * H + 4 * g) * 4u; }
+    __device__ __forceinline__ void load(const uint8_t *wg, int k0, uint32_t off) {
+        v[0] = ldg<f32x4>(wg + 4 * k0 + off);
+        v[1] = ldg<f32x4>(wg + 4 * k0 + 64 + off);
+    }
+    __device__ __forceinline__ void get(int, float (&f)[8]) const {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) f[k] = v[k / 4][k % 4];
+    }
+};
+template <>
+struct RmW<MOE_WG_F16> {
+    u32x2 v[2];
+    static __device__ __forceinline__ uint32_t offset(int H, int e, int g) { return ((uint32_t)e * H + 4 * g) * 2u; }
+    __device__ __forceinline__ void load(const uint8_t *wg, int k0, uint32_t off) {
+        v[0] = ldg<u32x2>(wg + 2 * k0 + off);
+        v[1] = ldg<u32x2>(wg + 2 * k0 + 32 + off);
+    }
+    __device__ __forceinline__ void get(int, float (&f)[8]) const {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) f[k] = (float)__builtin_bit_cast(f16x2, (uint32_t)v[k / 4][k % 4 / 2])[k % 2];
+    }
+};
+template <>
+struct RmW<MOE_WG_IQ4_XS> {
+    u32x2 hdr;
+    uint32_t q;
+    // a row is whole 16-byte pieces (1088 or 272 bytes), so the low bits are the lane's place in
+    // its sub-block's 16 qs bytes
+    static __device__ __forceinline__ uint32_t offset(int H, int e, int g) {
+        return (uint32_t)e * (H / QK * SB_BYTES) + 4u * (uint32_t)g;
+    }
+    __device__ __forceinline__ void load(const uint8_t *wg, int k0, uint32_t off) {
+        const uint8_t *blk = wg + k0 / QK * SB_BYTES;
+        hdr = ldg<u32x2>(blk + (off & ~15u));
+        q = ldg<uint32_t>(blk + 8 + 16 * (k0 % QK / 32) + off);
+    }
+    __device__ __forceinline__ void get(int k0, float (&f)[8]) const {
+        const float dl = sub_scale(hdr, k0 % QK / 32), off = -128.0f * dl;
+        uint32_t b[2];
+        kv_biased8(q, b[0], b[1]);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) f[k] = __builtin_fmaf(ubyte(b[k / 4], k % 4), dl, off); // (b - 128) dl, exact
+    }
+};
+
+template <int RB, int NW>
+struct RmShape { // RB x RB MFMA blocks of 16 x 16 per wave
+    static constexpr int TILE = 16 * RB, THREADS = 64 * NW;
+    static constexpr size_t SMEM = ((size_t)NW * TILE * TILE + NW * TILE + TILE) * 4;
+};
+
+template <int H, int WT, int RB, int NW, int ND>
+__global__ __launch_bounds__(64 * NW, NW / 4) void k_router_gemm(RouterGemvArgs a) {
+    using S = RmShape<RB, NW>;
+    constexpr int TILE = S::TILE, KW = H / NW, NST = KW / 32, DEPTH = ND < NST ? ND : NST;
+    static_assert(KW % 32 == 0 && H % QK == 0 && NST % DEPTH == 0, "whole turns of the ring per wave");
+    extern __shared__ float rm_smem[];
+    float *red = rm_smem, *s_ss = red + NW * TILE * TILE, *s_inv = s_ss + NW * TILE;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = lane & 15, g = lane >> 4;
+    const int M = a.M, E = a.E;
+    // workgroup w runs on XCD w % 8: the expert tiles of one token tile on one XCD, so its x rows
+    // come from memory once
+    const int nct = (E + TILE - 1) / TILE, w = (int)blockIdx.x;
+    const int rt = 8 * ((w >> 3) / nct) + (w & 7), ct = (w >> 3) % nct;
+    const int t0 = rt * TILE, e0 = ct * TILE;
+    if (t0 >= M) return;
+    // this lane's rows as byte offsets on the wave-uniform x (of the tile) and Wg plus the stage's
+    // K (tokens and experts past the end repeat the last)
+    const uint8_t *xt = (const uint8_t *)(a.x + (size_t)t0 * H), *wg = (const uint8_t *)a.wg;
+    uint32_t xo[RB], wo[RB];
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+        xo[r] = (uint32_t)(min(16 * r + i, M - 1 - t0) * H + 4 * g) * 4u;
+        wo[r] = RmW<WT>::offset(H, min(e0 + 16 * r + i, E - 1), g);
+    }
+    struct Stage {
+        f32x4 x[RB][2];
+        RmW<WT> w[RB];
+    } st[DEPTH];
+    auto issue = [&](Stage &s, int k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            s.x[r][0] = ldg<f32x4>(xt + 4 * k0 + xo[r]);
+            s.x[r][1] = ldg<f32x4>(xt + 4 * k0 + 64 + xo[r]);
+            s.w[r].load(wg, k0, wo[r]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    f32x4 tot[RB][RB], ss[RB];
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+        ss[r] = f32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int c = 0; c < RB; ++c) tot[r][c] = f32x4{0, 0, 0, 0};
+    }
+    auto compute = [&](const Stage &s, int k0) __attribute__((always_inline)) {
+        float wf[RB][8];
+#pragma unroll
+        for (int r = 0; r < RB; ++r) s.w[r].get(k0, wf[r]);
+        f32x4 acc[RB][RB];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+#pragma unroll
+                for (int c = 0; c < RB; ++c)
+                    acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(s.x[r][k / 4][k % 4], wf[c][k],
+                                                                     k ? acc[r][c] : f32x4{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+#pragma unroll
+            for (int c = 0; c < RB; ++c) tot[r][c] += acc[r][c];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) ss[r][k % 4] = __builtin_fmaf(s.x[r][k / 4][k % 4], s.x[r][k / 4][k % 4], ss[r][k % 4]);
+        }
+    };
+    // the loop stays rolled, one turn of the ring an iteration (unrolled over all stages the
+    // compiler kept hundreds of operands live and spilled); requests past the last stage re-read it
+    const int kw = wv * KW;
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; ++d) issue(st[d], kw + 32 * d);
+#pragma unroll 1
+    for (int k0 = kw; k0 < kw + KW; k0 += 32 * DEPTH) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            issue(st[(d + DEPTH - 1) % DEPTH], min(k0 + 32 * (d + DEPTH - 1), kw + KW - 32));
+            compute(st[d], k0 + 32 * d);
+        }
+    }
+    // partial blocks and sums of squares to LDS (C: row 4 g + n, column i), then each logit summed
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+#pragma unroll
+        for (int c = 0; c < RB; ++c)
+#pragma unroll
+            for (int n = 0; n < 4; ++n) red[(wv * TILE + 16 * r + 4 * g + n) * TILE + 16 * c + i] = tot[r][c][n];
+        float q = (ss[r][0] + ss[r][1]) + (ss[r][2] + ss[r][3]);
+        q += __shfl_xor(q, 16);
+        q += __shfl_xor(q, 32);
+        if (g == 0) s_ss[wv * TILE + 16 * r + i] = q;
+    }
+    __syncthreads();
+    if (tid < TILE) {
+        double q = 0.0;
+#pragma unroll
+        for (int v = 0; v < NW; ++v) q += (double)s_ss[v * TILE + tid];
+        s_inv[tid] = a.rmsnorm ? (float)(1.0 / sqrt(q * (1.0 / H) + 1e-6)) : 1.0f;
+    }
+    __syncthreads();
+    for (int o = tid; o < TILE * TILE; o += S::THREADS) {
+        const int r = o / TILE, c = o % TILE;
+        double v = 0.0;
+#pragma unroll
+        for (int p = 0; p < NW; ++p) v += (double)red[p * TILE * TILE + o];
+        if (t0 + r < M && e0 + c < E) a.logits[(size_t)(t0 + r) * E + e0 + c] = (float)(v * (double)s_inv[r]);
+    }
+}
+
+template <int H, int WT, int RB, int NW, int ND>
+static void launch_router_gemm_t(const RouterGemvArgs &a, hipStream_t st) {
+    using S = RmShape<RB, NW>;
+    const int nrt = ((a.M + S::TILE - 1) / S::TILE + 7) / 8 * 8, nct = (a.E + S::TILE - 1) / S::TILE;
+    hipLaunchKernelGGL((k_router_gemm<H, WT, RB, NW, ND>), dim3((unsigned)(nrt * nct)), dim3(S::THREADS), S::SMEM, st, a);
+}
+
 template <int H, int TM, int WT>
 static void launch_router_gemv_t(const RouterGemvArgs &a, hipStream_t st) {
     const dim3 grid((unsigned)((a.E + RG_WAVES - 1) / RG_WAVES), (unsigned)((a.M + TM - 1) / TM));
     hipLaunchKernelGGL((k_router_gemv<H, TM, WT>), grid, dim3(64 * RG_WAVES), 0, st, a);
 }
 
+template <int RB, int NW>
+static int rm_tiles(const RouterGemvArgs &a) {
+    using S = RmShape<RB, NW>;
+    return ((a.M + S::TILE - 1) / S::TILE) * ((a.E + S::TILE - 1) / S::TILE);
+}
+
+// One row per wave while its waves fit the 1,024 SIMDs (M <= 16 at E = 256, 64 at E = 64), then
+// the matrix product with the smallest tile that fills the 256 CUs at most twice.  Measured (us,
+// f32 gate, E = 256, graph replays; E = 128, M = 16 / 64: 6.6 / 11.4 by rows, 9.0 / 9.1 by tiles):
+//     M                  8     16     64    256    512   1000   2048   4096
+//     one row per wave  6.7    6.8   20.8   73     142    276    558   1112
+//     16 x 16           8.0    9.2    9.2    9.4  17.3   33.2   65.1    127
+//     32 x 32          13.8   15.2   18.2   18.3  18.5   19.1   35.5   68.1
+//     64 x 64          41.2   41.5   43.3   43.7  43.7   43.4   43.9   45.8
+// Every 16 x 16 or 64 x 64 workgroup has a CU to itself and takes the same time whatever M is:
+// its rows lie 8 KB apart, so the rows of a load share an L2 channel.
 template <int H, int WT>
 static void launch_router_gemv_w(const RouterGemvArgs &a, hipStream_t st) {
     // a wave's tokens past M repeat the last one: at small M fewer tokens per wave
     if (a.M == 1) launch_router_gemv_t<H, 1, WT>(a, st);
     else if (a.M == 2) launch_router_gemv_t<H, 2, WT>(a, st);
-    else launch_router_gemv_t<H, 4, WT>(a, st);
+    else if (a.E * ((a.M + 3) / 4) <= RG_GEMV_MAX_WAVES) launch_router_gemv_t<H, 4, WT>(a, st);
+    else if (rm_tiles<1, 8>(a) <= 512) launch_router_gemm_t<H, WT, 1, 8, 8>(a, st);
+    else if (rm_tiles<2, 8>(a) <= 512) launch_router_gemm_t<H, WT, 2, 8, 2>(a, st);
+    else launch_router_gemm_t<H, WT, 4, 4, 2>(a, st);
 }
 
 template <int H>

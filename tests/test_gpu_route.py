@@ -160,6 +160,24 @@ def test_router_gemv_small_shape(gpu, orc, M):
         c.close()
 
 
+# The edges of launch_router_gemv_w's rule and of the tiles: one row per wave / 16 x 16 (M = 16,
+# 17 at E = 256; 64, 65 at E = 64), 16 x 16 / 32 x 32 (512 tiles of 16), 32 x 32 / 64 x 64 (512 tiles of 32), one token or
+# expert more or less than a tile, fewer experts than a tile, both hidden sizes.
+@pytest.mark.parametrize("H_,E_,M", [(2048, 256, 16), (2048, 256, 17), (2048, 64, 64), (2048, 64, 65),
+                                     (2048, 8, 515), (2048, 200, 95),
+                                     (2048, 256, 512), (2048, 256, 513), (2048, 72, 1700), (2048, 256, 2049),
+                                     (512, 9, 33), (512, 129, 1000), (512, 256, 2081)])
+@pytest.mark.parametrize("dense", [None, np.float32, np.float16])
+def test_router_gemm_tile_edges(gpu, orc, H_, E_, M, dense):
+    log(f"router gemm E={E_} H={H_} M={M} {dense}")
+    c = gpu.Context(H_, 512 if H_ == 2048 else 256, E_, 1, 16, gpu.W_RENORM)
+    try:
+        got = _router_gemv_case(gpu, orc, c, E_, H_, M, 0x52473000 + M, M % 2 == 0, dense=dense)
+    finally:
+        c.close()
+    assert got.shape == (M, E_)
+
+
 def test_router_gemv_outputs_and_errors(gpu, orc, ctx):
     import torch
     log("router gemv: logits-only, ids-only, bad flags")
