@@ -64,6 +64,28 @@
 
 namespace moe {
 
+// The stack's codebook lookups keep the three-perm form (two perms over the table halves and a
+// third choosing per byte on index bit 3): they run in the waits between the phases, where the
+// shorter form of moe_device.hpp gains nothing (252 us per 40-layer token either way), and in the
+// activation-routed kernel, which spills, its extra temporaries cost (415 -> 431 us).
+// (x & 0x04040404) | 0x03020100 in one v_bitop3_b32 (truth table 0xEA = (a & b) | c).
+__device__ __forceinline__ uint32_t stk_sel_bit3(uint32_t x) {
+    return __builtin_amdgcn_bitop3_b32(x, 0x04040404u, 0x03020100u, 0xEA);
+}
+template <uint32_t T0, uint32_t T1, uint32_t T2, uint32_t T3>
+__device__ __forceinline__ uint32_t stk_lookup16(uint32_t idx_lo3, uint32_t sel_bit3) {
+    const uint32_t lo = __builtin_amdgcn_perm(T1, T0, idx_lo3), hi = __builtin_amdgcn_perm(T3, T2, idx_lo3);
+    return __builtin_amdgcn_perm(hi, lo, sel_bit3);
+}
+__device__ __forceinline__ void stk_kv_biased8(uint32_t q, uint32_t &lo, uint32_t &hi) {
+    lo = stk_lookup16<KVB0, KVB1, KVB2, KVB3>(q & 0x07070707u, stk_sel_bit3(q >> 1));
+    hi = stk_lookup16<KVB0, KVB1, KVB2, KVB3>((q >> 4) & 0x07070707u, stk_sel_bit3(q >> 5));
+}
+__device__ __forceinline__ void stk_kv_signed8(uint32_t q, uint32_t &lo, uint32_t &hi) {
+    lo = stk_lookup16<KVS0, KVS1, KVS2, KVS3>(q & 0x07070707u, stk_sel_bit3(q >> 1));
+    hi = stk_lookup16<KVS0, KVS1, KVS2, KVS3>((q >> 4) & 0x07070707u, stk_sel_bit3(q >> 5));
+}
+
 // Per-phase timeline (a build with -DMOE_STACK_TRACE, libmoe680m_trace.so; moe_stack_trace):
 // lane 0 of the named wave stores the 100 MHz device clock (s_memrealtime, one clock for every
 // CU) at each event of each layer into trace[(workgroup * n_layers + layer) * STK_TRACE_EV +
@@ -875,14 +897,14 @@ __global__ __launch_bounds__(64 * STK_WAVES) void k_decode_stack(StackArgs a) {
         for (int st = 0; st < STA; ++st) {
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
-                kv_signed8(aq1[st][d], ak1[st][2 * d], ak1[st][2 * d + 1]);
-                kv_signed8(aq3[st][d], ak3[st][2 * d], ak3[st][2 * d + 1]);
+                stk_kv_signed8(aq1[st][d], ak1[st][2 * d], ak1[st][2 * d + 1]);
+                stk_kv_signed8(aq3[st][d], ak3[st][2 * d], ak3[st][2 * d + 1]);
             }
             as1[st] = sub_scale(header(hA1[st]), ib1);
             as3[st] = sub_scale(header(hA3[st]), ib1);
         }
-        kv_signed8(saq[0], sak[0], sak[1]);
-        kv_signed8(saq[1], sak[2], sak[3]);
+        stk_kv_signed8(saq[0], sak[0], sak[1]);
+        stk_kv_signed8(saq[1], sak[2], sak[3]);
         sas = sub_scale(header(hSA), sbg & 7);
         // ... and the results as well, so that the work is not sunk below the next barrier
         // either
@@ -900,16 +922,16 @@ __global__ __launch_bounds__(64 * STK_WAVES) void k_decode_stack(StackArgs a) {
         asm volatile("" : "+v"(aq1[st]), "+v"(aq3[st]), "+v"(hd0), "+v"(hd1));
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
-            kv_signed8(aq1[st][d], ak1[st][2 * d], ak1[st][2 * d + 1]);
-            kv_signed8(aq3[st][d], ak3[st][2 * d], ak3[st][2 * d + 1]);
+            stk_kv_signed8(aq1[st][d], ak1[st][2 * d], ak1[st][2 * d + 1]);
+            stk_kv_signed8(aq3[st][d], ak3[st][2 * d], ak3[st][2 * d + 1]);
         }
         as1[st] = sub_scale(header(hA1[st]), ib1);
         as3[st] = sub_scale(header(hA3[st]), ib1);
     };
     auto decode_a_shared = [&]() __attribute__((always_inline)) {
         asm volatile("" : "+v"(saq));
-        kv_signed8(saq[0], sak[0], sak[1]);
-        kv_signed8(saq[1], sak[2], sak[3]);
+        stk_kv_signed8(saq[0], sak[0], sak[1]);
+        stk_kv_signed8(saq[1], sak[2], sak[3]);
         sas = sub_scale(header(hSA), sbg & 7);
     };
 
@@ -921,10 +943,10 @@ __global__ __launch_bounds__(64 * STK_WAVES) void k_decode_stack(StackArgs a) {
 #pragma unroll
         for (int st = 0; st < STB; ++st) {
 #pragma unroll
-            for (int d = 0; d < 4; ++d) kv_biased8(bq[st][d], bk[st][2 * d], bk[st][2 * d + 1]);
+            for (int d = 0; d < 4; ++d) stk_kv_biased8(bq[st][d], bk[st][2 * d], bk[st][2 * d + 1]);
             bs[st] = sub_scale(header(hB[st]), ibB);
         }
-        kv_biased8(sbq, sbk[0], sbk[1]);
+        stk_kv_biased8(sbq, sbk[0], sbk[1]);
         sbs = sub_scale(header(hSBr), ccB & 7);
 #pragma unroll
         for (int st = 0; st < STB; ++st)
@@ -971,7 +993,7 @@ __global__ __launch_bounds__(64 * STK_WAVES) void k_decode_stack(StackArgs a) {
         if (rg_type == MOE_WG_IQ4_XS) {
             asm volatile("" : "+v"(rq[0]), "+v"(rgh));
 #pragma unroll
-            for (int d = 0; d < 4; ++d) kv_signed8(rq[0][d], rkv[2 * d], rkv[2 * d + 1]);
+            for (int d = 0; d < 4; ++d) stk_kv_signed8(rq[0][d], rkv[2 * d], rkv[2 * d + 1]);
             rsc = sub_scale(rgh, g1 & 7);
 #pragma unroll
             for (int e = 0; e < 8; ++e) asm volatile("" : "+v"(rkv[e]));

@@ -51,39 +51,58 @@ constexpr uint32_t KVS1 = 0xCFu | (0xDDu << 8) | (0xEAu << 16) | (0xF6u << 24);
 constexpr uint32_t KVS2 = 0x01u | (0x0Du << 8) | (0x19u << 16) | (0x26u << 24);
 constexpr uint32_t KVS3 = 0x35u | (0x45u << 8) | (0x59u << 16) | (0x71u << 24);
 
-// Four nibble indices (bits 0..3 of each byte, upper bits ignored by the masks below)
-// -> four table bytes.  v_perm_b32 picks bytes 0..7 of {S0:S1}; two perms cover table
-// halves 0..7 and 8..15 and a third chooses per byte on index bit 3.
+// Four 4-bit indices, one per byte -> four table bytes.  v_perm_b32 picks bytes 0..7 of {S0:S1}
+// by selectors 0..7; selector 8 + k gives the sign of byte 2k + 1 replicated (k < 4), 12 gives
+// 0x00 and 13..15 give 0xFF -- bytes known from the table alone.  So one perm over table half 0..7
+// on the index and one over half 8..15 on the index with bit 3 flipped each return a table byte
+// for one half of the indices and a known byte for the other: with every entry stored as
+// its value XOR what the other perm returns there, the XOR of the two is the table byte.  Two perms
+// and three 2-cycle ops (and, xor, xor) per four weights; the three-perm form with a select on
+// bit 3 took 22 to 25 cycles where this takes 16 to 18 (on gfx950 v_perm_b32, like every VOP3 and
+// conversion measured, issues in 4.4 cycles a wave, v_and/v_xor/v_lshrrev in 2.4).
+constexpr uint32_t table_byte(uint32_t w0, uint32_t w1, int i) { return ((i < 4 ? w0 : w1) >> (8 * (i & 3))) & 0xFFu; }
+struct XorTable {
+    uint32_t t[4]; // stored words of entries 0..3, 4..7, 8..11, 12..15
+};
+constexpr XorTable xor_table(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3) {
+    uint32_t lo[8] = {}, hi[8] = {}; // stored bytes of the two halves
+    for (int i = 7; i >= 0; --i) {
+        // what the other half's perm returns for selector 8 + i (its bytes 2i + 1 > i, known by now;
+        // for i = 0 byte 1)
+        const uint32_t ch = i == 4 ? 0x00u : i > 4 ? 0xFFu : (hi[2 * i + 1] & 0x80u) ? 0xFFu : 0x00u;
+        const uint32_t cl = i == 4 ? 0x00u : i > 4 ? 0xFFu : (lo[2 * i + 1] & 0x80u) ? 0xFFu : 0x00u;
+        lo[i] = table_byte(w0, w1, i) ^ ch;
+        hi[i] = table_byte(w2, w3, i) ^ cl;
+    }
+    XorTable x{};
+    for (int i = 0; i < 4; ++i) {
+        x.t[0] |= lo[i] << (8 * i);
+        x.t[1] |= lo[4 + i] << (8 * i);
+        x.t[2] |= hi[i] << (8 * i);
+        x.t[3] |= hi[4 + i] << (8 * i);
+    }
+    return x;
+}
+
+// idx: four indices 0..15, one per byte (upper bits clear).
 template <uint32_t T0, uint32_t T1, uint32_t T2, uint32_t T3>
-__device__ __forceinline__ uint32_t lookup16(uint32_t idx_lo3, uint32_t sel_bit3) {
-    uint32_t lo = __builtin_amdgcn_perm(T1, T0, idx_lo3);
-    uint32_t hi = __builtin_amdgcn_perm(T3, T2, idx_lo3);
-    return __builtin_amdgcn_perm(hi, lo, sel_bit3);
+__device__ __forceinline__ uint32_t lookup16(uint32_t idx) {
+    constexpr XorTable X = xor_table(T0, T1, T2, T3);
+    uint32_t flip; // in asm: the compiler makes (q & m) ^ 8 a v_bitop3 (4.4 cycles) instead of this v_xor (2.4)
+    asm("v_xor_b32 %0, %1, %2" : "=v"(flip) : "s"(0x08080808u), "v"(idx));
+    return __builtin_amdgcn_perm(X.t[1], X.t[0], idx) ^ __builtin_amdgcn_perm(X.t[3], X.t[2], flip);
 }
 
 // qs dword q (4 bytes = weights j..j+3 low nibbles, j+16..j+19 high nibbles).
 // Returns biased codebook bytes for the low nibbles (lo) and the high nibbles (hi).
-// (x & 0x04040404) | 0x03020100 in one v_bitop3_b32 (truth table 0xEA = (a & b) | c).
-__device__ __forceinline__ uint32_t sel_bit3(uint32_t x) {
-    return __builtin_amdgcn_bitop3_b32(x, 0x04040404u, 0x03020100u, 0xEA);
-}
-
 __device__ __forceinline__ void kv_biased8(uint32_t q, uint32_t &lo, uint32_t &hi) {
-    uint32_t a_lo = q & 0x07070707u;
-    uint32_t s_lo = sel_bit3(q >> 1);
-    uint32_t a_hi = (q >> 4) & 0x07070707u;
-    uint32_t s_hi = sel_bit3(q >> 5);
-    lo = lookup16<KVB0, KVB1, KVB2, KVB3>(a_lo, s_lo);
-    hi = lookup16<KVB0, KVB1, KVB2, KVB3>(a_hi, s_hi);
+    lo = lookup16<KVB0, KVB1, KVB2, KVB3>(q & 0x0F0F0F0Fu);
+    hi = lookup16<KVB0, KVB1, KVB2, KVB3>((q >> 4) & 0x0F0F0F0Fu);
 }
 
 __device__ __forceinline__ void kv_signed8(uint32_t q, uint32_t &lo, uint32_t &hi) {
-    uint32_t a_lo = q & 0x07070707u;
-    uint32_t s_lo = sel_bit3(q >> 1);
-    uint32_t a_hi = (q >> 4) & 0x07070707u;
-    uint32_t s_hi = sel_bit3(q >> 5);
-    lo = lookup16<KVS0, KVS1, KVS2, KVS3>(a_lo, s_lo);
-    hi = lookup16<KVS0, KVS1, KVS2, KVS3>(a_hi, s_hi);
+    lo = lookup16<KVS0, KVS1, KVS2, KVS3>(q & 0x0F0F0F0Fu);
+    hi = lookup16<KVS0, KVS1, KVS2, KVS3>((q >> 4) & 0x0F0F0F0Fu);
 }
 
 __device__ __forceinline__ float ubyte(uint32_t v, int i) {
