@@ -74,16 +74,25 @@ __device__ __forceinline__ uint32_t stk_sel_bit3(uint32_t x) {
 }
 template <uint32_t T0, uint32_t T1, uint32_t T2, uint32_t T3>
 __device__ __forceinline__ uint32_t stk_lookup16(uint32_t idx_lo3, uint32_t sel_bit3) {
-    const uint32_t lo = __builtin_amdgcn_perm(T1, T0, idx_lo3), hi = __builtin_amdgcn_perm(T3, T2, idx_lo3);
+    uint32_t lo = __builtin_amdgcn_perm(T1, T0, idx_lo3);
+    uint32_t hi = __builtin_amdgcn_perm(T3, T2, idx_lo3);
     return __builtin_amdgcn_perm(hi, lo, sel_bit3);
 }
 __device__ __forceinline__ void stk_kv_biased8(uint32_t q, uint32_t &lo, uint32_t &hi) {
-    lo = stk_lookup16<KVB0, KVB1, KVB2, KVB3>(q & 0x07070707u, stk_sel_bit3(q >> 1));
-    hi = stk_lookup16<KVB0, KVB1, KVB2, KVB3>((q >> 4) & 0x07070707u, stk_sel_bit3(q >> 5));
+    uint32_t a_lo = q & 0x07070707u;
+    uint32_t s_lo = stk_sel_bit3(q >> 1);
+    uint32_t a_hi = (q >> 4) & 0x07070707u;
+    uint32_t s_hi = stk_sel_bit3(q >> 5);
+    lo = stk_lookup16<KVB0, KVB1, KVB2, KVB3>(a_lo, s_lo);
+    hi = stk_lookup16<KVB0, KVB1, KVB2, KVB3>(a_hi, s_hi);
 }
 __device__ __forceinline__ void stk_kv_signed8(uint32_t q, uint32_t &lo, uint32_t &hi) {
-    lo = stk_lookup16<KVS0, KVS1, KVS2, KVS3>(q & 0x07070707u, stk_sel_bit3(q >> 1));
-    hi = stk_lookup16<KVS0, KVS1, KVS2, KVS3>((q >> 4) & 0x07070707u, stk_sel_bit3(q >> 5));
+    uint32_t a_lo = q & 0x07070707u;
+    uint32_t s_lo = stk_sel_bit3(q >> 1);
+    uint32_t a_hi = (q >> 4) & 0x07070707u;
+    uint32_t s_hi = stk_sel_bit3(q >> 5);
+    lo = stk_lookup16<KVS0, KVS1, KVS2, KVS3>(a_lo, s_lo);
+    hi = stk_lookup16<KVS0, KVS1, KVS2, KVS3>(a_hi, s_hi);
 }
 
 // Per-phase timeline (a build with -DMOE_STACK_TRACE, libmoe680m_trace.so; moe_stack_trace):
