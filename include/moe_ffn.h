@@ -84,18 +84,20 @@ typedef struct {
 } moe_layer_weights;
 
 /* Create a context on HIP device `device`: validates the shape, allocates every
- * workspace for m_max tokens and the one device copy of the weights that moe_bind_layer
+ * workspace for m_max tokens and the device copies of the weights that moe_bind_layer
  * fills (nothing is allocated later): n_layers x (E+1) x 3 matrices in the library's split
- * layout, which every kernel family reads.
+ * layout, which the decode kernels read, and -- with m_max > MOE_DECODE_MAX_M, and only where
+ * half of the device's memory stays free beside it -- the same in the tiled layout of the
+ * prefill GEMMs (which otherwise read the split one; the results are the same bit for bit).
  * Replaces the MoE slice of InferenceEngine::new (src/inference.rs:85-126) and the
  * scratch / routing regions of ArenaLayout::compute (src/memory.rs:32-96). */
 moe_status moe_create(int device, const moe_config *cfg, moe_ctx **out);
 moe_status moe_destroy(moe_ctx *ctx);
 
 /* Copy one layer's weights (device pointers, read only during this call) into the context's
- * split layout (same bytes, qs and headers of each super-block apart).  Synchronises the
+ * layouts (same bytes, qs and headers of each super-block apart).  Synchronises the
  * device: the caller's buffers may be freed when it returns.  Rebinding a layer replaces its
- * copy.
+ * copies.
  * Replaces LayerWeights::from_registry (src/memory.rs:227-291). */
 moe_status moe_bind_layer(moe_ctx *ctx, int layer, const moe_layer_weights *lw);
 

@@ -233,6 +233,49 @@ hipError_t launch_repack_split(const void *src, uint64_t src_stride, const void 
     return hipGetLastError();
 }
 
+// The prefill GEMMs' copy of a matrix of `rows` rows (a multiple of 16) of sbr super-blocks:
+//     [rows / 16 groups][2 sbr stages][4 sub-blocks][16 rows][16 qs bytes]
+//     [rows / 16 groups][sbr super-blocks][16 rows][8-byte header]
+// -- the natural layout's bytes in the order an MFMA wave's lanes take them, so each of its
+// loads is 1 KB of consecutive bytes in lane order (from the split copy, where a row's bytes are
+// together, neighbouring lanes read different rows and the load takes the address unit 64
+// cycles instead of 16).
+__global__ __launch_bounds__(256) void k_repack_tiled(const uint8_t *__restrict__ src, uint64_t src_stride,
+                                                      const uint8_t *__restrict__ shared, uint8_t *__restrict__ dst,
+                                                      uint64_t dst_stride, int E, uint32_t nsb, uint32_t sbr) {
+    const int e = blockIdx.y;
+    const uint8_t *m = (e == E) ? shared : src + (uint64_t)e * src_stride;
+    uint8_t *o = dst + (uint64_t)e * dst_stride;
+    // one thread per 8-byte word of the destination (a matrix is below 4 GB)
+    const uint32_t nq = nsb * 16;
+    for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < nq + nsb; t += gridDim.x * blockDim.x) {
+        uint32_t row, sb, off;
+        if (t < nq) {
+            const uint32_t half = t & 1, n = (t >> 1) & 15, g = (t >> 5) & 3, st = (t >> 7) % (2 * sbr), rg = (t >> 7) / (2 * sbr);
+            row = rg * 16 + n;
+            sb = st >> 1;
+            off = 8 + 16 * (4 * (st & 1) + g) + 8 * half;
+        } else {
+            const uint32_t u = t - nq;
+            row = (u >> 4) / sbr * 16 + (u & 15);
+            sb = (u >> 4) % sbr;
+            off = 0;
+        }
+        const uint64_t v = *reinterpret_cast<const uint64_t *>(m + ((uint64_t)row * sbr + sb) * SB_BYTES + off);
+        *reinterpret_cast<uint64_t *>(o + 8ull * t) = v;
+    }
+}
+
+hipError_t launch_repack_tiled(const void *src, uint64_t src_stride, const void *shared, void *dst,
+                               uint64_t dst_stride, int E, int rows, int cols, hipStream_t st) {
+    const uint32_t sbr = (uint32_t)(cols / QK), nsb = (uint32_t)rows * sbr;
+    const uint32_t blocks = (nsb * 17 + 255) / 256;
+    dim3 grid(blocks < 4096 ? blocks : 4096, (unsigned)(E + 1));
+    hipLaunchKernelGGL(k_repack_tiled, grid, dim3(256), 0, st, (const uint8_t *)src, src_stride,
+                       (const uint8_t *)shared, (uint8_t *)dst, dst_stride, E, nsb, sbr);
+    return hipGetLastError();
+}
+
 // One workgroup: thread 0 swaps the flags out; after an expired decode-stack wait, thread 0
 // clears the abort word and all threads zero the stack's control words and exchange sets (an error path: its speed does not
 // matter, and the usual call only reads and clears one word).

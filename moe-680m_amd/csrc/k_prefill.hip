@@ -334,22 +334,28 @@ __device__ __forceinline__ const T *uniform_ptr(const T *p) {
 }
 
 // Raw IQ4_XS data of one K stage (PF_KC = 128 K = 4 sub-blocks, half a super-block) for NR
-// 16-row weight groups, read from the split layout (k_repack_split): lane (g, n) gets the
-// header of row n and, in one 16-byte load, the 16 qs bytes of sub-block 4h + g of row n (h =
-// the stage's half of the super-block).  MFMA K-step ks of the stage then takes dword ks of
-// every lane's sub-block: lane group g supplies K positions 32 g + 8 ks .. + 7 of the stage (in
-// the 32-block permuted K order of xh), and its sub-block scale is the same in all 4 steps.
-// Stages live in a ring so each is requested a few stages ahead.
+// 16-row weight groups: lane (g, n) gets the header of row n and, in one 16-byte load, the 16 qs
+// bytes of sub-block 4h + g of row n (h = the stage's half of the super-block).  MFMA K-step ks of
+// the stage then takes dword ks of every lane's sub-block: lane group g supplies K positions 32 g
+// + 8 ks .. + 7 of the stage (in the 32-block permuted K order of xh), and its sub-block scale is
+// the same in all 4 steps.  Stages live in a ring so each is requested a few stages ahead.
+// TILED: from the tiled copy (k_repack_tiled), where the 1 KB of a load is contiguous and in lane
+// order; else from the split copy (k_repack_split; a context without the tiled one: moe_create), where
+// a row's bytes are together, so neighbouring lanes read rows 128 SBR bytes apart and the address
+// unit takes them one by one.  Measured, one layer, split -> tiled (us): M = 21 83.0 -> 77.7,
+// M = 512 (Zipf) 116 -> 109, M = 4096 467 -> 448.
+template <bool TILED>
 struct WRows {
-    const uint8_t *q; // qs of the group's first row (matrix base + row * SBR * 128)
-    const uint8_t *h; // header of the group's first row (header array + row * SBR * 8)
+    const uint8_t *q; // qs of the 16-row group: TILED, stage c at 1024 c; else its first row's
+    const uint8_t *h; // headers of the group: TILED, super-block s at 128 s; else its first row's
 };
 
-// Rows row0 .. row0 + 15 of a split matrix of `rows` rows and SBR super-blocks per row.
-template <int SBR>
-__device__ __forceinline__ WRows split_rows(const uint8_t *m, int rows, int row0) {
-    return WRows{uniform_ptr(m + (size_t)row0 * SBR * 128),
-                 uniform_ptr(m + (size_t)rows * SBR * 128 + (size_t)row0 * SBR * 8)};
+// Rows row0 .. row0 + 15 (row0 a multiple of 16) of a matrix of `rows` rows and SBR super-blocks
+// per row (both layouts: the qs of whole 16-row groups, then their headers).
+template <int SBR, bool TILED>
+__device__ __forceinline__ WRows<TILED> weight_rows(const uint8_t *m, int rows, int row0) {
+    return WRows<TILED>{uniform_ptr(m + (size_t)row0 * SBR * 128),
+                        uniform_ptr(m + (size_t)rows * SBR * 128 + (size_t)row0 * SBR * 8)};
 }
 
 template <int NR>
@@ -358,17 +364,18 @@ struct WStage {
     u32x4 q[NR];
 };
 
-template <int SBR, int NR>
-__device__ __forceinline__ void wstage_load(WStage<NR> &s, const WRows (&groups)[NR], int ch, int lane) {
-    const int sb = ch >> 1, h = ch & 1;
+template <int SBR, bool TILED, int NR>
+__device__ __forceinline__ void wstage_load(WStage<NR> &s, const WRows<TILED> (&groups)[NR], int ch, int lane) {
     // unsigned lane offsets (zero-extended) on wave-uniform bases that go through
     // readfirstlane: the loads then take an SGPR base and one 32-bit lane offset
+    const int sb = ch >> 1, h = ch & 1;
     const uint32_t n = (uint32_t)(lane & 15), g = (uint32_t)(lane >> 4);
-    const uint32_t oh = n * (SBR * 8u), oq = n * (SBR * 128u) + 16u * g;
+    const uint32_t oh = TILED ? 8u * n : n * (SBR * 8u), oq = TILED ? 16u * (uint32_t)lane : n * (SBR * 128u) + 16u * g;
+    const size_t bh = TILED ? (size_t)sb * 128 : (size_t)sb * 8, bq = TILED ? (size_t)ch * 1024 : (size_t)sb * 128 + 64 * h;
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
-        s.hdr[r] = ldg<u32x2>(uniform_ptr(groups[r].h + (size_t)sb * 8) + oh);
-        s.q[r] = ldg<u32x4>(uniform_ptr(groups[r].q + (size_t)sb * 128 + 64 * h) + oq);
+        s.hdr[r] = ldg<u32x2>(uniform_ptr(groups[r].h + bh) + oh);
+        s.q[r] = ldg<u32x4>(uniform_ptr(groups[r].q + bq) + oq);
     }
 }
 
@@ -387,12 +394,15 @@ __device__ __forceinline__ void wstage_bc(const WStage<NR> &s, int ch, int g, co
 // the row's headers (row_dmax_load, issued with the first loads of the work item); row_shift
 // takes the maximum over the row's four lane groups and returns F = 2^(24 - s_n) for bc_pair
 // and P = 2^s_n for the epilogue.  A row whose d are all zero gets F = 2^127 (its B are 0).
-template <int SBR>
-__device__ __forceinline__ u32x2 row_dmax_load(const WRows &w, int n, int g) {
-    if constexpr (SBR == 1) {
+template <int SBR, bool TILED>
+__device__ __forceinline__ u32x2 row_dmax_load(const WRows<TILED> &w, int n, int g) {
+    static_assert(SBR == 1 || SBR == 2 || SBR == 4 || SBR == 8, "one or two headers per lane group");
+    if constexpr (TILED) {
+        const uint32_t o = 8u * (uint32_t)n + 128u * (uint32_t)(g % SBR);
+        return u32x2{ldg<uint32_t>(w.h + o), SBR == 8 ? ldg<uint32_t>(w.h + 512u + o) : 0u};
+    } else if constexpr (SBR == 1) {
         return u32x2{ldg<uint32_t>(w.h + (uint32_t)n * 8u), 0u};
     } else {
-        static_assert(SBR == 2 || SBR == 4 || SBR == 8, "one or two headers per lane group");
         const u32x4 v = ldg<u32x4>(w.h + (uint32_t)n * (SBR * 8u) + 16u * (uint32_t)(g % (SBR / 2)));
         return u32x2{v[0], v[2]};
     }
@@ -475,19 +485,19 @@ __device__ __forceinline__ void alt_prio(int sp, int st) {
 }
 
 // Weight ring of RD register stages: the prologue requests stages 0..RD-2.
-template <int NCH, int RD, int SBR, int NR>
-__device__ __forceinline__ void wring_prologue(WStage<NR> (&ws)[RD], const WRows (&rows)[NR], int lane) {
+template <int NCH, int RD, int SBR, bool TILED, int NR>
+__device__ __forceinline__ void wring_prologue(WStage<NR> (&ws)[RD], const WRows<TILED> (&rows)[NR], int lane) {
 #pragma unroll
     for (int c = 0; c < RD - 1; ++c) {
-        if (c < NCH) wstage_load<SBR>(ws[c], rows, c, lane);
+        if (c < NCH) wstage_load<SBR, TILED>(ws[c], rows, c, lane);
         __builtin_amdgcn_sched_barrier(0);
     }
 }
 
 // stage_a(c) moves chunk c of A into LDS; chunk 0 is expected in LDS on entry (its loads were
 // issued before the weight ring's, so waiting for them did not wait for the weights).
-template <int NCH, int RD, int SBR, int NR, int MT, typename StageA>
-__device__ __forceinline__ void gemm_resident(WStage<NR> (&ws)[RD], const WRows (&rows)[NR], const float (&F)[NR],
+template <int NCH, int RD, int SBR, bool TILED, int NR, int MT, typename StageA>
+__device__ __forceinline__ void gemm_resident(WStage<NR> (&ws)[RD], const WRows<TILED> (&rows)[NR], const float (&F)[NR],
                                               const _Float16 *As, int n, int g, int sp, f32x4 (&acc)[MT][NR],
                                               StageA stage_a) {
     constexpr int KCH = pf_kch<NCH, MT>();
@@ -507,7 +517,7 @@ __device__ __forceinline__ void gemm_resident(WStage<NR> (&ws)[RD], const WRows 
         // keep the scheduler from moving loads across stages: each stage's weights are
         // requested RD-1 stages ahead, in the order they are consumed
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (ch + RD - 1 < NCH) wstage_load<SBR>(ws[(ch + RD - 1) % RD], rows, ch + RD - 1, n + 16 * g);
+        if constexpr (ch + RD - 1 < NCH) wstage_load<SBR, TILED>(ws[(ch + RD - 1) % RD], rows, ch + RD - 1, n + 16 * g);
         __builtin_amdgcn_sched_barrier(0);
     });
 }
@@ -517,8 +527,8 @@ __device__ __forceinline__ void gemm_resident(WStage<NR> (&ws)[RD], const WRows 
 // columns; chunk boundaries (KCH even) fall at the same loop index for both.  Half-length
 // work items: gate/up's items then fill the 512 workgroup slots in three rounds of half
 // length instead of two full ones (at M = 512, ~1140 items against ~570 of twice the length).
-template <int NCH, int RD, int SBR, int NR, int MT, typename StageA>
-__device__ __forceinline__ void gemm_resident_split(WStage<NR> (&ws)[RD], const WRows (&rows)[NR],
+template <int NCH, int RD, int SBR, bool TILED, int NR, int MT, typename StageA>
+__device__ __forceinline__ void gemm_resident_split(WStage<NR> (&ws)[RD], const WRows<TILED> (&rows)[NR],
                                                     const float (&F)[NR], const _Float16 *As, int n, int g,
                                                     int p, f32x4 (&acc)[MT][NR], StageA stage_a) {
     constexpr int KCH = pf_kch<NCH, MT>();
@@ -538,7 +548,7 @@ __device__ __forceinline__ void gemm_resident_split(WStage<NR> (&ws)[RD], const 
         wstage_bc(ws[S], ch, g, F, b2, c2);
         stage_mfma<NR, MT, LK>(ws[S], b2, c2, As + (ch0 % KCH + p) * PF_KC, n, g, acc);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (c + RD - 1 < NC2) wstage_load<SBR>(ws[(c + RD - 1) % RD], rows, 2 * (c + RD - 1) + p, n + 16 * g);
+        if constexpr (c + RD - 1 < NC2) wstage_load<SBR, TILED>(ws[(c + RD - 1) % RD], rows, 2 * (c + RD - 1) + p, n + 16 * g);
         __builtin_amdgcn_sched_barrier(0);
     });
 }
@@ -602,7 +612,7 @@ __device__ __forceinline__ Tile tile_record(const Tile *tiles, int ti) {
     return Tile{(int32_t)v[0], (int32_t)v[1], (int32_t)v[2], 0};
 }
 
-template <int H, int I, bool SPLIT>
+template <int H, int I, bool SPLIT, bool TILED>
 __global__ __launch_bounds__(64 * PF_WAVES, 4) void k_pf_gate_up(PrefillArgs a) {
     constexpr int NGU = SPLIT ? PF_NGU : PF_NGU_WIDE;
     static_assert(NGU == 16 * PF_WAVES / (SPLIT ? 2 : 1), "16 columns per wave (pair)");
@@ -637,8 +647,8 @@ __global__ __launch_bounds__(64 * PF_WAVES, 4) void k_pf_gate_up(PrefillArgs a) 
     }
     lds_barrier();
     // Weights: rows c0 + n of W1 (gate) and W3 (up).
-    const WRows rows[2] = {split_rows<SBR>(expert_w(a.L.w1, a.L.s1, a.L.sw1, e, a.E), I, c0),
-                           split_rows<SBR>(expert_w(a.L.w3, a.L.s3, a.L.sw3, e, a.E), I, c0)};
+    const WRows<TILED> rows[2] = {weight_rows<SBR, TILED>(expert_w(a.L.w1, a.L.s1, a.L.sw1, e, a.E), I, c0),
+                           weight_rows<SBR, TILED>(expert_w(a.L.w3, a.L.s3, a.L.sw3, e, a.E), I, c0)};
 
     by_mtiles(nrows, [&](auto MTc) __attribute__((always_inline)) {
         constexpr int MT = decltype(MTc)::value;
@@ -673,15 +683,15 @@ __global__ __launch_bounds__(64 * PF_WAVES, 4) void k_pf_gate_up(PrefillArgs a) 
         // the rows' headers for their shifts after A and before the first weights (requested
         // ahead of A, their registers were reused by A's addressing and the A loads waited for
         // them; requested after the weights, the first stage would wait for all of those)
-        const u32x2 dq[2] = {row_dmax_load<SBR>(rows[0], n, g), row_dmax_load<SBR>(rows[1], n, g)};
+        const u32x2 dq[2] = {row_dmax_load<SBR, TILED>(rows[0], n, g), row_dmax_load<SBR, TILED>(rows[1], n, g)};
         if constexpr (SPLIT) {
 #pragma unroll
             for (int c = 0; c < RD - 1; ++c) {
-                if (c < NCH / 2) wstage_load<SBR>(ws[c], rows, 2 * c + p, lane);
+                if (c < NCH / 2) wstage_load<SBR, TILED>(ws[c], rows, 2 * c + p, lane);
                 __builtin_amdgcn_sched_barrier(0);
             }
         } else {
-            wring_prologue<NCH, RD, SBR>(ws, rows, lane);
+            wring_prologue<NCH, RD, SBR, TILED>(ws, rows, lane);
         }
         store_a(0, PER);
         float F[2], P[2];
@@ -708,7 +718,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 4) void k_pf_gate_up(PrefillArgs a) 
         constexpr int NE = 4 * MT, NOWN = SPLIT ? NE / 2 : NE;
         const int el0 = SPLIT && p ? NE / 2 : 0;
         if constexpr (SPLIT) {
-            gemm_resident_split<NCH, RD, SBR, 2, MT>(ws, rows, F, As, n, g, p, acc, stage_a);
+            gemm_resident_split<NCH, RD, SBR, TILED, 2, MT>(ws, rows, F, As, n, g, p, acc, stage_a);
             __builtin_amdgcn_s_setprio(0);
             lds_barrier();
             float *red = reinterpret_cast<float *>(As);
@@ -725,7 +735,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 4) void k_pf_gate_up(PrefillArgs a) 
 #pragma unroll
                     for (int r = 0; r < 2; ++r) acc[el / 4][r][el % 4] += red[((cw * NE + el) * 2 + r) * 64 + lane];
         } else {
-            gemm_resident<NCH, RD, SBR, 2, MT>(ws, rows, F, As, n, g, (wv >> 2) & 1, acc, stage_a);
+            gemm_resident<NCH, RD, SBR, TILED, 2, MT>(ws, rows, F, As, n, g, (wv >> 2) & 1, acc, stage_a);
             __builtin_amdgcn_s_setprio(0);
             lds_barrier(); // s_inv
         }
@@ -766,7 +776,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 4) void k_pf_gate_up(PrefillArgs a) 
 
 // ---------------------------------------------------------------- down
 // NGU: the column width of h's scale blocks (the gate/up item width).
-template <int H, int I, int NGU>
+template <int H, int I, int NGU, bool TILED>
 __global__ __launch_bounds__(64 * PF_WAVES, 4) void k_pf_down(PrefillArgs a) {
     constexpr int NTW = 2, NCH = I / PF_KC;
     constexpr int SBR = I / QK;
@@ -788,7 +798,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 4) void k_pf_down(PrefillArgs a) {
     const int n = lane & 15, g = lane >> 4;
     const int r0 = item * PF_ND + wv * 32; // this wave's output rows r0 .. r0+31
     const uint8_t *w2 = expert_w(a.L.w2, a.L.s2, a.L.sw2, e, a.E);
-    const WRows rows[NTW] = {split_rows<SBR>(w2, H, r0), split_rows<SBR>(w2, H, r0 + 16)};
+    const WRows<TILED> rows[NTW] = {weight_rows<SBR, TILED>(w2, H, r0), weight_rows<SBR, TILED>(w2, H, r0 + 16)};
 
     by_mtiles(nrows, [&](auto MTc) __attribute__((always_inline)) {
         constexpr int MT = decltype(MTc)::value;
@@ -819,10 +829,10 @@ __global__ __launch_bounds__(64 * PF_WAVES, 4) void k_pf_down(PrefillArgs a) {
         }
         // the rows' headers for their shifts after the h rows, before the weights (requested
         // first, their registers were reused by the h rows' addressing and the h loads waited)
-        const u32x2 dq[NTW] = {row_dmax_load<SBR>(rows[0], n, g), row_dmax_load<SBR>(rows[1], n, g)};
+        const u32x2 dq[NTW] = {row_dmax_load<SBR, TILED>(rows[0], n, g), row_dmax_load<SBR, TILED>(rows[1], n, g)};
         constexpr int RD = 4; // weight ring depth: three stages ahead
         WStage<NTW> ws[RD];
-        wring_prologue<NCH, RD, SBR>(ws, rows, lane);
+        wring_prologue<NCH, RD, SBR, TILED>(ws, rows, lane);
 #pragma unroll
         for (int j = 0; j < IPT; ++j) {
             const int it = j * 64 * PF_WAVES + tid;
@@ -861,7 +871,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 4) void k_pf_down(PrefillArgs a) {
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int t = 0; t < NTW; ++t) acc[i][t] = f32x4{0, 0, 0, 0};
-        gemm_resident<NCH, RD, SBR, NTW, MT>(ws, rows, F, As, n, g, -1, acc, [](int) {});
+        gemm_resident<NCH, RD, SBR, TILED, NTW, MT>(ws, rows, F, As, n, g, -1, acc, [](int) {});
 
         // epilogue: v = c * w * 2^-s_row * 2^s_n * acc per slot row (s_n: the weight row's shift); each row's 32 values of this
         // wave are stored as f16 times a power of two 2^sh that puts their max in
@@ -949,7 +959,7 @@ __global__ __launch_bounds__(256) void k_pf_combine(PrefillArgs a) {
     }
 }
 
-template <int H, int I>
+template <int H, int I, bool TILED>
 static hipError_t launch_prefill_t(const BucketArgs &b, const PfCountArgs &c, const PrefillArgs &a, hipStream_t st,
                                    KernelTimer *T) {
     // the chain's own fill: count (routing first with logits), then place + prep
@@ -972,13 +982,13 @@ static hipError_t launch_prefill_t(const BucketArgs &b, const PfCountArgs &c, co
     const bool split = a.M <= PF_SPLIT_MAX_M;
     {
         TimedLaunch tl(T, MOE_K_PREFILL_GATE_UP, st);
-        if (split) hipLaunchKernelGGL((k_pf_gate_up<H, I, true>), dim3(I / PF_NGU, ntiles), dim3(64 * PF_WAVES), 0, st, a);
-        else hipLaunchKernelGGL((k_pf_gate_up<H, I, false>), dim3(I / PF_NGU_WIDE, ntiles), dim3(64 * PF_WAVES), 0, st, a);
+        if (split) hipLaunchKernelGGL((k_pf_gate_up<H, I, true, TILED>), dim3(I / PF_NGU, ntiles), dim3(64 * PF_WAVES), 0, st, a);
+        else hipLaunchKernelGGL((k_pf_gate_up<H, I, false, TILED>), dim3(I / PF_NGU_WIDE, ntiles), dim3(64 * PF_WAVES), 0, st, a);
     }
     {
         TimedLaunch tl(T, MOE_K_PREFILL_DOWN, st);
-        if (split) hipLaunchKernelGGL((k_pf_down<H, I, PF_NGU>), dim3(H / PF_ND, ntiles), dim3(64 * PF_WAVES), 0, st, a);
-        else hipLaunchKernelGGL((k_pf_down<H, I, PF_NGU_WIDE>), dim3(H / PF_ND, ntiles), dim3(64 * PF_WAVES), 0, st, a);
+        if (split) hipLaunchKernelGGL((k_pf_down<H, I, PF_NGU, TILED>), dim3(H / PF_ND, ntiles), dim3(64 * PF_WAVES), 0, st, a);
+        else hipLaunchKernelGGL((k_pf_down<H, I, PF_NGU_WIDE, TILED>), dim3(H / PF_ND, ntiles), dim3(64 * PF_WAVES), 0, st, a);
     }
     {
         TimedLaunch tl(T, MOE_K_PREFILL_COMBINE, st);
@@ -989,8 +999,10 @@ static hipError_t launch_prefill_t(const BucketArgs &b, const PfCountArgs &c, co
 
 hipError_t launch_prefill(int H, int I, const BucketArgs &b, const PfCountArgs &c, const PrefillArgs &a,
                           hipStream_t st, KernelTimer *T) {
-    if (H == 2048 && I == 512) return launch_prefill_t<2048, 512>(b, c, a, st, T);
-    if (H == 512 && I == 256) return launch_prefill_t<512, 256>(b, c, a, st, T);
+    if (H == 2048 && I == 512)
+        return a.tiled ? launch_prefill_t<2048, 512, true>(b, c, a, st, T) : launch_prefill_t<2048, 512, false>(b, c, a, st, T);
+    if (H == 512 && I == 256)
+        return a.tiled ? launch_prefill_t<512, 256, true>(b, c, a, st, T) : launch_prefill_t<512, 256, false>(b, c, a, st, T);
     return hipErrorInvalidValue;
 }
 

@@ -20,9 +20,12 @@ using namespace moe;
 struct moe_ctx {
     int device = 0;
     moe_config cfg{};
-    std::vector<LayerPtrs> slayers; // the library's split copy of each bound layer (every kernel)
+    std::vector<LayerPtrs> slayers; // the library's split copy of each bound layer
+    std::vector<LayerPtrs> tlayers; // ... and its tiled copy, when there is one
     std::vector<char> bound;
-    uint8_t *spk = nullptr;         // [n_layers][E+1][W1|W3|W2] split layout: the one resident copy
+    uint8_t *spk = nullptr;         // [n_layers][E+1][W1|W3|W2] split layout (decode kernels)
+    uint8_t *tpk = nullptr;         // the same matrices tiled (prefill GEMMs): m_max > MOE_DECODE_MAX_M and
+                                    // ample device memory, else null and the GEMMs read spk
     void *arena = nullptr; // one device allocation, carved below
     size_t arena_bytes = 0;
     uint32_t *flags = nullptr;   // [0] sticky device flags, [1] the decode stack's abort word
@@ -134,6 +137,7 @@ moe_status moe_create(int device, const moe_config *cfg, moe_ctx **out) {
     c->device = device;
     c->cfg = *cfg;
     c->slayers.resize(cfg->n_layers);
+    c->tlayers.resize(cfg->n_layers);
     c->bound.assign(cfg->n_layers, 0);
     c->hrouters.assign(cfg->n_layers, StackRouter{nullptr, 0u, 0u});
 
@@ -179,8 +183,8 @@ moe_status moe_create(int device, const moe_config *cfg, moe_ctx **out) {
         off += align_up(p.bytes, 256);
     }
     {
-        // every kernel family reads the library's own split copy of each bound layer
-        // (k_repack_split); the caller's buffers are not read after moe_bind_layer returns
+        // the kernels read the library's own copies of each bound layer (k_repack_split,
+        // k_repack_tiled); the caller's buffers are not read after moe_bind_layer returns
         const size_t mat = (size_t)H * I / QK * SB_BYTES;
         const size_t sbytes = (size_t)cfg->n_layers * E1 * 3 * mat;
         he = hipMalloc((void **)&c->spk, sbytes);
@@ -190,6 +194,13 @@ moe_status moe_create(int device, const moe_config *cfg, moe_ctx **out) {
             return fail(MOE_ENOMEM, "moe_create: hipMalloc(%zu) for the weight copies: %s", sbytes,
                         hipGetErrorString(he));
         }
+        // the tiled copy only where half of the device's memory stays free beside it: without it
+        // the prefill GEMMs read the split copy, 4 to 8 % more slowly
+        size_t mfree = 0, mtotal = 0;
+        if (cfg->m_max > MOE_DECODE_MAX_M && hipMemGetInfo(&mfree, &mtotal) == hipSuccess &&
+            mfree >= sbytes + mtotal / 2 && hipMalloc((void **)&c->tpk, sbytes) != hipSuccess)
+            c->tpk = nullptr;
+        (void)hipGetLastError();
     }
     c->xtag_words = STK_CTL_WORDS + 2 * (size_t)cfg->n_layers * stack_layer_words(H, I);
     he = hipMemset(c->flags, 0, 256);
@@ -200,6 +211,7 @@ moe_status moe_create(int device, const moe_config *cfg, moe_ctx **out) {
     if (he == hipSuccess) he = hipMemset(c->xtag, 0, c->xtag_words * 4);
     if (he == hipSuccess) he = hipDeviceSynchronize();
     if (he != hipSuccess) {
+        if (c->tpk) (void)hipFree(c->tpk);
         if (c->spk) (void)hipFree(c->spk);
         (void)hipFree(c->arena);
         delete c;
@@ -228,6 +240,7 @@ moe_status moe_destroy(moe_ctx *ctx) {
     (void)hipSetDevice(ctx->device);
     (void)hipDeviceSynchronize();
     timer_free(ctx->timer);
+    if (ctx->tpk) (void)hipFree(ctx->tpk);
     if (ctx->spk) (void)hipFree(ctx->spk);
     hipError_t he = hipFree(ctx->arena);
     delete ctx;
@@ -263,23 +276,35 @@ moe_status moe_bind_layer(moe_ctx *ctx, int layer, const moe_layer_weights *lw) 
     hipError_t he;
     {
         const size_t es = 3 * mat;
-        uint8_t *base = ctx->spk + (size_t)layer * (E + 1) * es;
+        const size_t off = (size_t)layer * (E + 1) * es;
+        uint8_t *base = ctx->spk + off;
         he = launch_repack_split(L.w1, L.s1, L.sw1, base, es, E, I, H, nullptr);
         if (he == hipSuccess) he = launch_repack_split(L.w3, L.s3, L.sw3, base + mat, es, E, I, H, nullptr);
         if (he == hipSuccess) he = launch_repack_split(L.w2, L.s2, L.sw2, base + 2 * mat, es, E, H, I, nullptr);
+        if (ctx->tpk) {
+            uint8_t *t = ctx->tpk + off;
+            if (he == hipSuccess) he = launch_repack_tiled(L.w1, L.s1, L.sw1, t, es, E, I, H, nullptr);
+            if (he == hipSuccess) he = launch_repack_tiled(L.w3, L.s3, L.sw3, t + mat, es, E, I, H, nullptr);
+            if (he == hipSuccess) he = launch_repack_tiled(L.w2, L.s2, L.sw2, t + 2 * mat, es, E, H, I, nullptr);
+        }
         if (he == hipSuccess) he = hipDeviceSynchronize();
-        if (he != hipSuccess) return hip_fail(he, "moe_bind_layer: repacking into the split layout");
-        LayerPtrs S;
-        S.w1 = base;
-        S.w3 = base + mat;
-        S.w2 = base + 2 * mat;
-        S.s1 = S.s3 = S.s2 = es;
-        S.sw1 = base + (size_t)E * es;
-        S.sw3 = S.sw1 + mat;
-        S.sw2 = S.sw1 + 2 * mat;
+        if (he != hipSuccess) return hip_fail(he, "moe_bind_layer: repacking the weights");
+        auto ptrs_at = [&](uint8_t *b) {
+            LayerPtrs S;
+            S.w1 = b;
+            S.w3 = b + mat;
+            S.w2 = b + 2 * mat;
+            S.s1 = S.s3 = S.s2 = es;
+            S.sw1 = b + (size_t)E * es;
+            S.sw3 = S.sw1 + mat;
+            S.sw2 = S.sw1 + 2 * mat;
+            return S;
+        };
+        const LayerPtrs S = ptrs_at(base);
         he = hipMemcpy(ctx->dlayers + layer, &S, sizeof(LayerPtrs), hipMemcpyHostToDevice);
         if (he != hipSuccess) return hip_fail(he, "moe_bind_layer: copying the layer table");
         ctx->slayers[layer] = S;
+        if (ctx->tpk) ctx->tlayers[layer] = ptrs_at(ctx->tpk + off);
     }
     ctx->bound[layer] = 1;
     return ok();
@@ -448,7 +473,8 @@ static moe_status ffn_call(const char *fn, moe_ctx *ctx, int layer, const float 
     b.tile_max = tile_max_for(M, E + 1);
     b.flags = ctx->flags;
     PrefillArgs p{};
-    p.L = ctx->slayers[layer];
+    p.tiled = ctx->tpk != nullptr;
+    p.L = p.tiled ? ctx->tlayers[layer] : ctx->slayers[layer];
     p.x = x;
     p.xh = ctx->xh;
     p.xinv = ctx->xinv;

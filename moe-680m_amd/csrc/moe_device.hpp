@@ -253,7 +253,7 @@ __device__ __forceinline__ float subblock_dot_mix(const uint32_t (&kv)[8], const
 }
 
 // ---------------------------------------------------------------- split weight layout
-// The library's one resident copy of every bound matrix (k_repack_split): for a matrix of
+// The library's copy of every bound matrix for the decode kernels (k_repack_split): for a matrix of
 // `rows` rows of SBR super-blocks each,
 //     [rows * SBR qs blocks of 128 bytes, row-major] [rows * SBR headers of 8 bytes, same order]
 // -- the bytes of the GGML layout (136 per super-block) split in two, so that every 16-byte

@@ -98,9 +98,9 @@ constexpr int PF_SLOT_RANK_BITS = 23; // a slot's expert above these bits
 constexpr int PF_CNT_COPIES = 8;      // striped bucket counters (one per XCD)
 constexpr int PF_SLOT_COPY_SHIFT = 20; // its counter copy at bits 20..22, its rank below: ranks < 9 * 65535 < 2^20
 
-// Prefill reads the split copy of a layer (k_repack_split), as the decode kernels do.
 struct PrefillArgs {
-    LayerPtrs L;
+    LayerPtrs L;         // the layer's tiled copy (k_repack_tiled), or its split copy (k_repack_split)
+    int tiled;
     const float *x;
     _Float16 *xh;        // [M][H] f16: x (normalised if requested) * s_t, K permuted in 32-blocks
     float *xinv;         // [M] 1 / s_t (s_t a power of two)
@@ -195,9 +195,12 @@ struct TimedLaunch {
 };
 
 hipError_t launch_dequant(const void *blocks, uint64_t n_sb, float *out, hipStream_t st);
-// Decode-stack copy of a layer: per matrix, the 128-byte qs of every super-block, then its
+// The decode kernels' copy of a layer: per matrix, the 128-byte qs of every super-block, then its
 // 8-byte headers, same order (k_repack_split).
 hipError_t launch_repack_split(const void *src, uint64_t src_stride, const void *shared, void *dst,
+                               uint64_t dst_stride, int E, int rows, int cols, hipStream_t st);
+// The prefill GEMMs' copy of a layer (k_repack_tiled).
+hipError_t launch_repack_tiled(const void *src, uint64_t src_stride, const void *shared, void *dst,
                                uint64_t dst_stride, int E, int rows, int cols, hipStream_t st);
 hipError_t launch_gen_iq4xs(void *dst, uint64_t n, uint64_t seed, uint64_t first, hipStream_t st);
 hipError_t launch_gen_normal(float *dst, uint64_t n, uint64_t seed, uint64_t first, float mean,

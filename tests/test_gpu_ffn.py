@@ -141,6 +141,27 @@ def test_prefill_flags(gpu, orc, full):
         assert err <= TOL_PREFILL
 
 
+def test_prefill_from_split_copy(gpu, full):
+    """A context whose weights leave too little device memory free for the tiled copy runs the
+    prefill GEMMs from the split copy: the same y bit for bit, every tile height and both item
+    widths (the same weights, bound to both contexts)."""
+    import torch
+    ctx, layer = full
+    total = torch.cuda.mem_get_info()[1]
+    n_layers = int(0.35 * total) // gpu.layer_bytes(H, I, E)
+    big = gpu.Context(H, I, E, n_layers, 1100, ctx.wmode)
+    try:
+        big.bind_packed(n_layers - 1, layer.dev)
+        for M in (9, 40, 300, 768, 769, 1100):
+            x = gpu.gen_normal(M * H, 3500 + M).view(M, H)
+            ids, w = ctx.router_topk(gpu.gen_logits(M, E, 3501 + M, kind=1, param=1.1))
+            y0, y1 = ctx.ffn(0, x, ids, w), big.ffn(n_layers - 1, x, ids, w)
+            torch.cuda.synchronize()
+            assert torch.equal(y0, y1), M
+    finally:
+        big.close()
+
+
 @pytest.fixture(scope="module")
 def full_renorm(gpu, full):
     """The moe-680m layer of `full` in a context with BASELINE's weight convention."""
