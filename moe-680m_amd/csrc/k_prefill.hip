@@ -10,7 +10,7 @@
 //            max|x| in [2^14, 2^15), stored as f16 with K permuted inside 32-blocks (the
 //            order the weight nibbles arrive in, see below); 1/s_t kept per token -- run in
 //            the same launch as the slot placement (k_pf_place), which does not need it;
-//   gate_up: per (tile, 64 gate/up column pairs; 128 when M > 768) a workgroup of 8 waves,
+//   gate_up: per (tile, 64 gate/up column pairs; 128 when M > 512) a workgroup of 8 waves,
 //            two per CU; the tile's token rows (gathered -- the reference's kernel skipped
 //            this gather) are resident in LDS one 64 KB chunk of K at a time and shared by the
 //            8 waves; each wave decodes 16 W1 rows and 16 W3 rows (with 64 columns, two waves
@@ -455,11 +455,11 @@ __device__ __forceinline__ void stage_mfma(const WStage<NR> &s0, const uint32_t 
 // wave's in-order vmcnt waits then never hold a use behind a later prefetch); the ring runs
 // on across chunks.  Fully unrolled: with a rolled loop the compiler's vmcnt bookkeeping
 // merges at the loop head and waits for every prefetch in flight.
-// Stages per resident chunk for MT M-tiles (16*MT rows x KCH*PF_KC halves = 64 KB), and the
+// Stages per resident chunk for MT M-tiles (16*MT rows x KCH*PF_KC halves <= 64 KB), and the
 // chunk's LDS row stride in halves: +16 B per row, so the 16 rows of an A fragment read hit
 // 16 different bank groups.
 template <int NCH, int MT>
-constexpr int pf_kch() { return NCH < 16 / MT ? NCH : 16 / MT; }
+constexpr int pf_kch() { return NCH < 16 / MT ? NCH : MT == 3 ? 4 : 16 / MT; }
 template <int NCH, int MT>
 constexpr int pf_ldsr() { return pf_kch<NCH, MT>() * PF_KC + 8; }
 constexpr int PF_AS_HALVES = PF_BM * (4 * PF_KC + 8); // the largest chunk (64 rows x 520)
@@ -553,7 +553,7 @@ __device__ __forceinline__ void gemm_resident_split(WStage<NR> (&ws)[RD], const 
     });
 }
 
-// A tile holds up to PF_BM slots of one expert and runs as 1, 2 or 4 M-tiles of 16 rows (one
+// A tile holds up to PF_BM slots of one expert and runs as 1 to 4 M-tiles of 16 rows (one
 // instantiation each, picked per workgroup, so every inner loop is straight-line code).  Full
 // PF_BM tiles come first in the list, remainders after: the long work items start first and
 // the short ones fill in.  64-row tiles, not 128: every wave reads each A fragment from LDS
@@ -563,7 +563,8 @@ __device__ __forceinline__ void gemm_resident_split(WStage<NR> (&ws)[RD], const 
 template <typename F>
 __device__ __forceinline__ void by_mtiles(int nrows, F f) {
     static_assert(PF_BM == 64 && PF_SMALL_MAX == 32, "tile classes");
-    if (nrows > PF_SMALL_MAX) f(std::integral_constant<int, 4>{});
+    if (nrows > 48) f(std::integral_constant<int, 4>{});
+    else if (nrows > PF_SMALL_MAX) f(std::integral_constant<int, 3>{});
     else if (nrows > 16) f(std::integral_constant<int, 2>{});
     else f(std::integral_constant<int, 1>{});
 }
@@ -574,7 +575,7 @@ __device__ __forceinline__ void by_mtiles(int nrows, F f) {
 // tile on one XCD -- the tile's token rows (gate/up) or h rows (down) come from HBM once and
 // are L2 hits for its other items -- and consecutive tiles on consecutive XCDs, in dispatch
 // order.  Used for the wide items of large M (measured, M = 4096: gate/up 310 -> 292 us, down
-// 189 -> 176 us); at M <= 768 the rows of all the tiles stay in the memory-side cache anyway
+// 189 -> 176 us); at M <= 512 the rows of all the tiles stay in the memory-side cache anyway
 // and one tile's items spread over the eight XCDs run faster (M = 512: 124 against 132 us).
 template <int ITEMS, bool GROUP>
 __device__ __forceinline__ void xcd_tile_item(int &tile, int &item) {

@@ -16,11 +16,14 @@ constexpr int PF_BM = 64;  // prefill big-tile rows (token slots of one expert)
 constexpr int PF_SMALL_MAX = 32; // remainders of at most this many slots are listed as small tiles
 // h columns per prefill gate/up work item, and per hmax block: 64 (two waves per 16 columns,
 // alternate K stages: half-length items, which fill the last round of workgroup slots better)
-// for M <= PF_SPLIT_MAX_M, else 128 (one wave per 16 columns: fewer items to stage A for).
-// Measured (H 2048, I 512): split 121.8 / wide 127.4 us at M = 512; 184.6 / 175.8 at 1024.
+// for M <= PF_SPLIT_MAX_M, else 128 (one wave per 16 columns: fewer items to stage A for, a tile's
+// items on one XCD).  Measured (H 2048, I 512, one layer, 64 / 128 columns, us): E = 256 uniform
+// M = 256 128.1 / 127.2, 512 154.5 / 142.3, 640 156.1 / 150.8; Zipf 256 82.4 / 80.4, 512 105.1 /
+// 108.4, 640 122.5 / 117.4; E = 128 uniform 150 80.7 / 82.5, 256 85.7 / 88.3, 512 107.9 / 104.9;
+// E = 64 256 72.0 / 74.0, 400 84.0 / 84.4, 512 92.6 / 88.9: above 512 every routing gains.
 constexpr int PF_NGU = 64;
 constexpr int PF_NGU_WIDE = 128;
-constexpr int PF_SPLIT_MAX_M = 768;
+constexpr int PF_SPLIT_MAX_M = 512;
 
 struct DecodeArgs {
     LayerPtrs L;          // split copy of the layer (k_repack_split)

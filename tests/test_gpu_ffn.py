@@ -141,6 +141,28 @@ def test_prefill_flags(gpu, orc, full):
         assert err <= TOL_PREFILL
 
 
+@pytest.mark.parametrize("M", [512, 513])
+@pytest.mark.parametrize("n", [16, 17, 32, 33, 48, 49, 64, 65])
+def test_prefill_tile_heights(gpu, orc, full, M, n):
+    """Expert 7 gets exactly n slots (the edges of the 1 to 4 M-tiles of 16 rows, and one slot more
+    than a full tile), the others what is left, at both sides of the item-width rule; checked on the
+    tokens of expert 7 and as many others."""
+    import torch
+    ctx, layer = full
+    x = gpu.gen_normal(M * H, 3700 + n).view(M, H)
+    logits = gpu.gen_logits(M, E, 3800 + n)
+    logits[:, 7] = -30.0
+    logits[:n, 7] = 30.0
+    ids, w = ctx.router_topk(logits)
+    y = ctx.ffn(0, x, ids, w, rmsnorm=True)
+    torch.cuda.synchronize()
+    ids_h = ids.cpu().numpy()
+    assert (ids_h[:, :8] == 7).sum() == n
+    t = np.r_[0:n, M - n:M]
+    ref = orc.moe_ffn(layer.host(), x.cpu().numpy()[t], ids_h[t], w.cpu().numpy()[t], 1.0 / 9, flags=2)
+    check_errs(y.cpu().numpy()[t], ref, False)
+
+
 def test_prefill_from_split_copy(gpu, full):
     """A context whose weights leave too little device memory free for the tiled copy runs the
     prefill GEMMs from the split copy: the same y bit for bit, every tile height and both item
@@ -152,7 +174,7 @@ def test_prefill_from_split_copy(gpu, full):
     big = gpu.Context(H, I, E, n_layers, 1100, ctx.wmode)
     try:
         big.bind_packed(n_layers - 1, layer.dev)
-        for M in (9, 40, 300, 768, 769, 1100):
+        for M in (9, 40, 512, 513, 1100):
             x = gpu.gen_normal(M * H, 3500 + M).view(M, H)
             ids, w = ctx.router_topk(gpu.gen_logits(M, E, 3501 + M, kind=1, param=1.1))
             y0, y1 = ctx.ffn(0, x, ids, w), big.ffn(n_layers - 1, x, ids, w)
