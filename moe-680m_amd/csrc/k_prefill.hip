@@ -204,7 +204,7 @@ __device__ __forceinline__ void prep_token(const PrefillArgs &a, int t, int lane
 // The counters start at zero and k_pf_combine, the chain's last launch, zeroes them again.
 // The shared expert's bucket has no counter: token t's shared row is row t of it.
 constexpr int PF_COUNT_TOKENS = 8; // tokens per counting workgroup, one wave each (16: 6.3 against 5.1 us at M = 512; 4: 10.3 against 8.7 us at M = 4096)
-constexpr uint32_t PF_SLOT_HOLE = 0xFFFFFFFEu; // slot 8 of a token with no kept shared slot
+constexpr uint32_t PF_SLOT_HOLE = 0xFFFFFFFEu; // dropped slot 8 of a token with no kept shared slot
 
 template <bool ROUTE>
 __global__ __launch_bounds__(64 * PF_COUNT_TOKENS) void k_pf_count(PfCountArgs c) {
@@ -262,7 +262,9 @@ __global__ __launch_bounds__(64 * PF_COUNT_TOKENS) void k_pf_count(PfCountArgs c
     __syncthreads();
     if (tok && lane < SLOTS) {
         uint32_t info = 0xFFFFFFFFu;
-        if (routed) info = ((uint32_t)id << PF_SLOT_RANK_BITS) | (cp << PF_SLOT_COPY_SHIFT) | (base[id] + rank);
+        if (routed)
+            info = ((uint32_t)id << PF_SLOT_RANK_BITS) | (cp << PF_SLOT_COPY_SHIFT) | (base[id] + rank) |
+                   (lane == SLOTS - 1 && !ns ? PF_SLOT_NO_SHARED : 0u);
         else if (keep) info = ((uint32_t)c.E << PF_SLOT_RANK_BITS) | (uint32_t)t; // the shared slot
         else if (lane == SLOTS - 1 && !ns) info = PF_SLOT_HOLE;
         c.slot[(size_t)t * SLOTS + lane] = info;
@@ -304,19 +306,23 @@ __global__ __launch_bounds__(BF_THREADS) void k_pf_place(BucketArgs b, PfCountAr
     __syncthreads();
     bucket_lists(b, S, blk == 0);
     const int n = SLOTS * b.M, i0 = blk * PF_PLACE_SLOTS, i1 = min(i0 + PF_PLACE_SLOTS, n);
+    // token t's shared row, unused: a valid token index, weight 0
+    auto hole = [&](int t) __attribute__((always_inline)) {
+        const uint32_t q = S.rg[E1 - 1] + (uint32_t)t;
+        b.sorted_tok[q] = (uint16_t)t;
+        b.sorted_w[q] = 0.0f;
+    };
     for (int i = i0 + tid; i < i1; i += BF_THREADS) {
         const uint32_t info = ldg<uint32_t>(c.slot + i);
         const float wv = ldg<float>(c.w + i);
         const int t = i / SLOTS;
         uint32_t p = 0xFFFFFFFFu;
         if (info == PF_SLOT_HOLE) {
-            // the token's shared row, unused: a valid token index, weight 0
-            const uint32_t q = S.rg[E1 - 1] + (uint32_t)t;
-            b.sorted_tok[q] = (uint16_t)t;
-            b.sorted_w[q] = 0.0f;
+            hole(t);
         } else if (info != 0xFFFFFFFFu) {
+            if (info & PF_SLOT_NO_SHARED) hole(t);
             const uint32_t e = info >> PF_SLOT_RANK_BITS, k = (info >> PF_SLOT_COPY_SHIFT) & (PF_CNT_COPIES - 1u);
-            p = S.rg[e] + (e < (uint32_t)E1 - 1u ? cb[k * E1 + e] : 0u) + (info & ((1u << PF_SLOT_COPY_SHIFT) - 1u));
+            p = S.rg[e] + (e < (uint32_t)E1 - 1u ? cb[k * E1 + e] : 0u) + (info & (PF_SLOT_NO_SHARED - 1u));
             b.sorted_tok[p] = (uint16_t)t;
             b.sorted_w[p] = wv;
         }
@@ -768,7 +774,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 4) void k_pf_gate_up(PrefillArgs a) 
             if (m < nrows) {
                 float unused;
                 const float sc = pow2_scale(__builtin_bit_cast(float, rowmax[m]), &unused);
-                a.hh[(uint32_t)((row0 + m) * I + hcol)] = (_Float16)(hv[j] * sc); // < 2^31: 9 m_max I
+                a.hh[(uint32_t)((row0 + m) * I + hcol)] = (_Float16)(hv[j] * sc); // < 2^31: 10 m_max I
             }
         }
     });

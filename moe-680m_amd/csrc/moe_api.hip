@@ -32,14 +32,14 @@ struct moe_ctx {
     float *hbuf = nullptr;       // decode path h scratch [72][I]
     _Float16 *xh = nullptr;      // [m_max][H]
     float *xinv = nullptr;       // [m_max]
-    _Float16 *hh = nullptr;      // [9 m_max][I]
-    float *hmax = nullptr;       // [9 m_max][I/PF_NGU]
-    _Float16 *part = nullptr;    // [9 m_max][H]
-    int8_t *pexp = nullptr;      // [9 m_max][H/32]
+    _Float16 *hh = nullptr;      // [10 m_max][I]
+    float *hmax = nullptr;       // [10 m_max][I/PF_NGU]
+    _Float16 *part = nullptr;    // [10 m_max][H]
+    int8_t *pexp = nullptr;      // [10 m_max][H/32]
     float *logits = nullptr;     // [m_max][E] router GEMV output when the caller gives none
     uint32_t *ranges = nullptr;  // [E+2]
-    uint16_t *stok = nullptr;    // [9 m_max]
-    float *sw = nullptr;         // [9 m_max]
+    uint16_t *stok = nullptr;    // [10 m_max]
+    float *sw = nullptr;         // [10 m_max]
     uint32_t *pos = nullptr;     // [m_max][9]
     uint32_t *chunk = nullptr;   // [ceil(m_max/64)][E+1]
     uint32_t *pcnt = nullptr;    // [PF_CNT_COPIES][E+1] the prefill chain's bucket counters (zero between calls)
@@ -143,7 +143,7 @@ moe_status moe_create(int device, const moe_config *cfg, moe_ctx **out) {
 
     const size_t mm = (size_t)cfg->m_max, E1 = (size_t)E + 1;
     const size_t nchunk = (mm + 63) / 64;
-    const size_t tmax = (size_t)tile_max_for((int)mm, (int)E1);
+    const size_t tmax = (size_t)tile_max_for(PF_ROWS_GIVEN * (int)mm, (int)E1);
     struct Part {
         void **dst;
         size_t bytes;
@@ -152,14 +152,14 @@ moe_status moe_create(int device, const moe_config *cfg, moe_ctx **out) {
         {(void **)&c->hbuf, decode_scratch_floats(H, I) * sizeof(float)},
         {(void **)&c->xh, mm * H * 2},
         {(void **)&c->xinv, mm * 4},
-        {(void **)&c->hh, SLOTS * mm * I * 2},
-        {(void **)&c->hmax, SLOTS * mm * (I / PF_NGU) * 4},
-        {(void **)&c->part, SLOTS * mm * H * 2},
-        {(void **)&c->pexp, SLOTS * mm * (H / 32)},
+        {(void **)&c->hh, PF_ROWS_GIVEN * mm * I * 2},
+        {(void **)&c->hmax, PF_ROWS_GIVEN * mm * (I / PF_NGU) * 4},
+        {(void **)&c->part, PF_ROWS_GIVEN * mm * H * 2},
+        {(void **)&c->pexp, PF_ROWS_GIVEN * mm * (H / 32)},
         {(void **)&c->logits, mm * (size_t)E * 4},
         {(void **)&c->ranges, (E1 + 1) * 4},
-        {(void **)&c->stok, SLOTS * mm * 2},
-        {(void **)&c->sw, SLOTS * mm * 4},
+        {(void **)&c->stok, PF_ROWS_GIVEN * mm * 2},
+        {(void **)&c->sw, PF_ROWS_GIVEN * mm * 4},
         {(void **)&c->pos, mm * SLOTS * 4},
         {(void **)&c->chunk, nchunk * E1 * 4},
         {(void **)&c->pcnt, (size_t)PF_CNT_COPIES * E1 * 4},
@@ -470,7 +470,7 @@ static moe_status ffn_call(const char *fn, moe_ctx *ctx, int layer, const float 
     b.pos = ctx->pos;
     b.chunk_cnt = ctx->chunk;
     b.tiles = ctx->tiles;
-    b.tile_max = tile_max_for(M, E + 1);
+    b.tile_max = tile_max_for((logits ? PF_ROWS_ROUTED : PF_ROWS_GIVEN) * M, E + 1);
     b.flags = ctx->flags;
     PrefillArgs p{};
     p.tiled = ctx->tpk != nullptr;

@@ -76,8 +76,8 @@ struct BucketArgs {
     const float *w;
     int M, E1; // E1 = n_experts + 1 buckets
     uint32_t *ranges;     // [E1+1]
-    uint16_t *sorted_tok; // [9M]
-    float *sorted_w;      // [9M]
+    uint16_t *sorted_tok; // [9M] (moe_bucket_fill), [rows] (prefill: PF_ROWS_*)
+    float *sorted_w;      // as sorted_tok
     uint32_t *pos;        // [M][9] or null
     uint32_t *chunk_cnt;  // workspace: ceil(M/64) * E1 chunk counts
     Tile *tiles;          // [tile_max]: full tiles, big remainders, small remainders, empty; or null
@@ -94,12 +94,18 @@ struct PfCountArgs {
     float *w;            // [M][9]
     int M, E, renorm;
     uint32_t *cnt;       // [E + 1] bucket counters: zero on entry (k_pf_combine zeroes them)
-    uint32_t *slot;      // [9M] (bucket << 23) | rank in the bucket, or ~0 for a dropped slot
+    uint32_t *slot;      // [9M] (bucket << 23) | copy | rank in the bucket, or ~0 for a dropped slot
     uint32_t *flags;
 };
 constexpr int PF_SLOT_RANK_BITS = 23; // a slot's expert above these bits
 constexpr int PF_CNT_COPIES = 8;      // striped bucket counters (one per XCD)
-constexpr int PF_SLOT_COPY_SHIFT = 20; // its counter copy at bits 20..22, its rank below: ranks < 9 * 65535 < 2^20
+constexpr int PF_SLOT_COPY_SHIFT = 20; // its counter copy at bits 20..22, its rank below: a token has one slot in a
+                                       // bucket, so ranks < 65535 < 2^16
+constexpr uint32_t PF_SLOT_NO_SHARED = 1u << 19; // slot 8 holds a routed expert and no slot the shared one
+// Rows of the sorted slot arrays per token: the routed slots' and one in the shared expert's bucket,
+// which every token has (k_pf_count) -- 9 for routed ids, up to 10 for given ids, whose nine may
+// all name routed experts.
+constexpr int PF_ROWS_ROUTED = SLOTS, PF_ROWS_GIVEN = SLOTS + 1;
 
 struct PrefillArgs {
     LayerPtrs L;         // the layer's tiled copy (k_repack_tiled), or its split copy (k_repack_split)
@@ -111,14 +117,14 @@ struct PrefillArgs {
     const float *sorted_w;
     const uint32_t *pos; // [M][9]
     const Tile *tiles;
-    _Float16 *hh;        // [9M][I] h = silu(g) * u as f16, sorted slot order: each PF_NGU-column
+    _Float16 *hh;        // [rows][I] h = silu(g) * u as f16, sorted slot order: each PF_NGU-column
                          // block scaled by the power of two of its max (hmax), K order of the
                          // down kernel's A (perm32_pos inside 32-column blocks)
-    float *hmax;         // [9M][I/PF_NGU] max |h| per row and PF_NGU-column block
-    _Float16 *part;      // [9M][H] c*w-scaled expert outputs in sorted slot order, as f16
+    float *hmax;         // [rows][I/PF_NGU] max |h| per row and PF_NGU-column block
+    _Float16 *part;      // [rows][H] c*w-scaled expert outputs in sorted slot order, as f16
                          // times 2^pexp per 32-column block; columns n and 16 + n of a block
                          // stored side by side
-    int8_t *pexp;        // [9M][H/32] those exponents
+    int8_t *pexp;        // [rows][H/32] those exponents
     float *y;
     int M, E, accumulate, rmsnorm, tile_max;
     float c;
@@ -238,8 +244,9 @@ constexpr int STK_LG_WORDS = 256;
 size_t stack_layer_words(int H, int I);
 
 // Tiles: the PF_BM-slot tiles of every expert, then each expert's remainder (above
-// PF_SMALL_MAX slots a big tile, else a small one): at most one remainder per expert.
-inline int tile_max_for(int M, int E1) { return (9 * M + PF_BM - 1) / PF_BM + E1; }
+// PF_SMALL_MAX slots a big tile, else a small one): the sum over the experts of ceil(n_e / PF_BM),
+// at most (rows + (PF_BM - 1) E1) / PF_BM.
+inline int tile_max_for(int rows, int E1) { return (rows + (PF_BM - 1) * E1) / PF_BM; }
 
 } // namespace moe
 

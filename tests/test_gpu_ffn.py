@@ -302,6 +302,30 @@ def test_duplicate_and_bad_ids_same_at_decode_and_prefill(gpu, orc, full):
     assert normwise_err(ref, ref0) <= 1e-12
 
 
+@pytest.mark.parametrize("M", [9, 57, 64, 130])
+def test_prefill_nine_routed_slots(gpu, orc, M):
+    """Given ids whose nine slots all name routed experts, none the shared one: such a token has nine
+    rows and an unused one in the shared expert's bucket, so a full context (M = m_max) where every
+    token is like that needs 10 M rows.  Then every third token only, the others routed as usual."""
+    import torch
+    E_ = 16
+    ctx = gpu.Context(512, 256, E_, 1, M, gpu.W_REF)
+    layer = Layer(gpu, orc, 31, 512, 256, E_)
+    ctx.bind_packed(0, layer.dev)
+    x = gpu.gen_normal(M * 512, 3900 + M).view(M, 512)
+    usual, w = ctx.router_topk(gpu.gen_logits(M, E_, 3901 + M))
+    usual_h, w_h = usual.cpu().numpy(), w.cpu().numpy()
+    nine = np.stack([np.random.default_rng(t).permutation(E_)[:9] for t in range(M)]).astype(np.uint16)
+    third = np.where(np.arange(M)[:, None] % 3 == 0, nine, usual_h)
+    for ids_h in (nine, third):
+        y = ctx.ffn(0, x, torch.from_numpy(ids_h).cuda(), w)
+        torch.cuda.synchronize()
+        assert ctx.device_flags() == 0
+        ref = orc.moe_ffn(layer.host(), x.cpu().numpy(), ids_h, w_h, 1.0 / 9)
+        check_errs(y.cpu().numpy(), ref, False)
+    ctx.close()
+
+
 def test_prefill_dropped_slots_skip_nonfinite_row0(gpu, orc, full):
     """Prefill (M = 16): token 0 routes to expert 0 in slot 0, so its partial output is
     expert-sorted row 0, and its activations are +inf (that row is non-finite).  Token 1 names
