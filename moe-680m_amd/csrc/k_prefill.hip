@@ -193,7 +193,7 @@ __device__ __forceinline__ void prep_token(const PrefillArgs &a, int t, int lane
 // and its partial are computed from that row alone, and the combine sums a token's slots in
 // slot order).  So the slots are ranked by an atomic counter per bucket rather than in token
 // order (moe_bucket_fill, the drop-in for build_expert_batches, keeps the token order), and the
-// fill takes two launches of many workgroups whatever M is:
+// fill takes two launches of many workgroups (few tokens: one launch, k_pf_fill_one):
 //   k_pf_count: one wave per token routes it (with logits, as k_router_topk) or reads its ids,
 //       applies the pair rule (an id above n_experts, or one its token named in an earlier slot,
 //       is dropped and flagged) and ranks each kept slot in its bucket: inside the workgroup by
@@ -206,31 +206,20 @@ __device__ __forceinline__ void prep_token(const PrefillArgs &a, int t, int lane
 constexpr int PF_COUNT_TOKENS = 8; // tokens per counting workgroup, one wave each (16: 6.3 against 5.1 us at M = 512; 4: 10.3 against 8.7 us at M = 4096)
 constexpr uint32_t PF_SLOT_HOLE = 0xFFFFFFFEu; // dropped slot 8 of a token with no kept shared slot
 
+// One token, by one wave (tok false: none), its ids and (ROUTE: routed here) weights in the lanes s < 9:
+// applies the pair rule and ranks the kept routed slots by the LDS counters hist.  slot_info: the
+// lane's slot word (c.slot) from the rank's start `first` in its bucket.
+struct CountedSlot {
+    int id;
+    uint32_t rank;
+    bool routed, keep, none; // none: the token keeps no shared slot
+};
 template <bool ROUTE>
-__global__ __launch_bounds__(64 * PF_COUNT_TOKENS) void k_pf_count(PfCountArgs c) {
-    // Routed experts: per-workgroup bucket counts in LDS first, then one global add per bucket
-    // the workgroup touched.  The shared expert's bucket takes no count: every token has one
-    // row in it, at rank t -- its kept shared slot, or (only when its ids name no valid shared
-    // slot) a hole row of weight 0 that no token reads back.  An add per shared slot would
-    // serialise M adds on one counter.
-    __shared__ uint32_t hist[MOE_MAX_EXPERTS + 1], base[MOE_MAX_EXPERTS + 1];
-    const int lane = threadIdx.x & 63, E1 = c.E + 1;
-    for (int e = threadIdx.x; e < E1; e += 64 * PF_COUNT_TOKENS) hist[e] = 0u;
-    __syncthreads();
-    const int t = blockIdx.x * PF_COUNT_TOKENS + (int)(threadIdx.x >> 6);
-    const bool tok = t < c.M; // whole waves
-    int id = 0;
-    if (tok) {
-        if constexpr (ROUTE) {
-            float wt;
-            route_wave<4>(c.logits + (size_t)t * c.E, c.E, c.renorm, lane, id, wt);
-            if (lane < SLOTS) {
-                c.ids[(size_t)t * SLOTS + lane] = (uint16_t)id;
-                c.w[(size_t)t * SLOTS + lane] = wt;
-            }
-        } else {
-            id = lane < SLOTS ? (int)c.ids[(size_t)t * SLOTS + lane] : 0;
-        }
+__device__ __forceinline__ CountedSlot count_token(const PfCountArgs &c, int t, bool tok, int lane, int id, float wt,
+                                                   uint32_t *hist) {
+    if (ROUTE && tok && lane < SLOTS) {
+        c.ids[(size_t)t * SLOTS + lane] = (uint16_t)id;
+        c.w[(size_t)t * SLOTS + lane] = wt;
     }
     // the pair rule for given ids; routed ids are E distinct indices and the shared id, so no
     // slot of theirs is dropped (ROUTE skips the check)
@@ -248,7 +237,36 @@ __global__ __launch_bounds__(64 * PF_COUNT_TOKENS) void k_pf_count(PfCountArgs c
     if (lane == 0 && (nb | nd))
         set_flag(c.flags, (nb ? (uint32_t)MOE_DEVFLAG_BAD_ID : 0u) | (nd ? (uint32_t)MOE_DEVFLAG_DUP_ID : 0u));
     const bool routed = keep && id != c.E;
-    uint32_t rank = routed ? atomicAdd(&hist[id], 1u) : 0u;
+    return CountedSlot{id, routed ? atomicAdd(&hist[id], 1u) : 0u, routed, keep, !ns};
+}
+__device__ __forceinline__ uint32_t slot_info(const CountedSlot &k, int E, int t, int lane, uint32_t copy, uint32_t first) {
+    if (k.routed)
+        return ((uint32_t)k.id << PF_SLOT_RANK_BITS) | (copy << PF_SLOT_COPY_SHIFT) | (first + k.rank) |
+               (lane == SLOTS - 1 && k.none ? PF_SLOT_NO_SHARED : 0u);
+    if (k.keep) return ((uint32_t)E << PF_SLOT_RANK_BITS) | (uint32_t)t; // the shared slot
+    return lane == SLOTS - 1 && k.none ? PF_SLOT_HOLE : 0xFFFFFFFFu;
+}
+
+template <bool ROUTE>
+__global__ __launch_bounds__(64 * PF_COUNT_TOKENS) void k_pf_count(PfCountArgs c) {
+    // Routed experts: per-workgroup bucket counts in LDS first, then one global add per bucket
+    // the workgroup touched.  The shared expert's bucket takes no count: every token has one
+    // row in it, at rank t -- its kept shared slot, or (only when its ids name no valid shared
+    // slot) a hole row of weight 0 that no token reads back.  An add per shared slot would
+    // serialise M adds on one counter.
+    __shared__ uint32_t hist[MOE_MAX_EXPERTS + 1], base[MOE_MAX_EXPERTS + 1];
+    const int lane = threadIdx.x & 63, E1 = c.E + 1;
+    for (int e = threadIdx.x; e < E1; e += 64 * PF_COUNT_TOKENS) hist[e] = 0u;
+    __syncthreads();
+    const int t = blockIdx.x * PF_COUNT_TOKENS + (int)(threadIdx.x >> 6);
+    const bool tok = t < c.M; // whole waves
+    int id = 0;
+    float wt = 0.0f;
+    if (tok) {
+        if constexpr (ROUTE) route_wave<4>(c.logits + (size_t)t * c.E, c.E, c.renorm, lane, id, wt);
+        else id = lane < SLOTS ? (int)c.ids[(size_t)t * SLOTS + lane] : 0;
+    }
+    const CountedSlot k = count_token<ROUTE>(c, t, tok, lane, id, wt, hist);
     __syncthreads();
     // counter copy blockIdx % 8 (the workgroup's XCD): a hot bucket's adds are spread over
     // eight addresses instead of queueing on one
@@ -260,15 +278,8 @@ __global__ __launch_bounds__(64 * PF_COUNT_TOKENS) void k_pf_count(PfCountArgs c
                     : 0u;
     }
     __syncthreads();
-    if (tok && lane < SLOTS) {
-        uint32_t info = 0xFFFFFFFFu;
-        if (routed)
-            info = ((uint32_t)id << PF_SLOT_RANK_BITS) | (cp << PF_SLOT_COPY_SHIFT) | (base[id] + rank) |
-                   (lane == SLOTS - 1 && !ns ? PF_SLOT_NO_SHARED : 0u);
-        else if (keep) info = ((uint32_t)c.E << PF_SLOT_RANK_BITS) | (uint32_t)t; // the shared slot
-        else if (lane == SLOTS - 1 && !ns) info = PF_SLOT_HOLE;
-        c.slot[(size_t)t * SLOTS + lane] = info;
-    }
+    if (tok && lane < SLOTS)
+        c.slot[(size_t)t * SLOTS + lane] = slot_info(k, c.E, t, lane, cp, k.routed ? base[k.id] : 0u);
 }
 
 // Slots per placing workgroup (one per thread) and tokens per prep workgroup (its first four
@@ -278,6 +289,28 @@ __global__ __launch_bounds__(64 * PF_COUNT_TOKENS) void k_pf_count(PfCountArgs c
 // 4096 slots and 16 tokens per workgroup).
 constexpr int PF_PLACE_SLOTS = 512; // slots per placing workgroup (1024: 12.8 against 12.3 us at M = 4096)
 constexpr int PF_PREP_TOKENS = 4; // tokens per prep workgroup, one wave each (16: 14.0 against 12.8 us at M = 4096)
+
+// Slot i's sorted token and weight, and its position.  cb: each counter copy's start inside the
+// buckets ([PF_CNT_COPIES][E1]; null: one copy).
+__device__ __forceinline__ void place_slot(const BucketArgs &b, const BucketScan &S, const uint32_t *cb, int i,
+                                           uint32_t info, float wv) {
+    const int t = i / SLOTS, E1 = b.E1;
+    uint32_t p = 0xFFFFFFFFu;
+    const bool kept = info < PF_SLOT_HOLE;
+    if (info == PF_SLOT_HOLE || (kept && (info & PF_SLOT_NO_SHARED))) {
+        // the token's shared row, unused: a valid token index, weight 0
+        const uint32_t q = S.rg[E1 - 1] + (uint32_t)t;
+        b.sorted_tok[q] = (uint16_t)t;
+        b.sorted_w[q] = 0.0f;
+    }
+    if (kept) {
+        const uint32_t e = info >> PF_SLOT_RANK_BITS, k = (info >> PF_SLOT_COPY_SHIFT) & (PF_CNT_COPIES - 1u);
+        p = S.rg[e] + (cb && e < (uint32_t)E1 - 1u ? cb[k * E1 + e] : 0u) + (info & (PF_SLOT_NO_SHARED - 1u));
+        b.sorted_tok[p] = (uint16_t)t;
+        b.sorted_w[p] = wv;
+    }
+    b.pos[i] = p;
+}
 
 template <int H>
 __global__ __launch_bounds__(BF_THREADS) void k_pf_place(BucketArgs b, PfCountArgs c, PrefillArgs a) {
@@ -306,28 +339,65 @@ __global__ __launch_bounds__(BF_THREADS) void k_pf_place(BucketArgs b, PfCountAr
     __syncthreads();
     bucket_lists(b, S, blk == 0);
     const int n = SLOTS * b.M, i0 = blk * PF_PLACE_SLOTS, i1 = min(i0 + PF_PLACE_SLOTS, n);
-    // token t's shared row, unused: a valid token index, weight 0
-    auto hole = [&](int t) __attribute__((always_inline)) {
-        const uint32_t q = S.rg[E1 - 1] + (uint32_t)t;
-        b.sorted_tok[q] = (uint16_t)t;
-        b.sorted_w[q] = 0.0f;
-    };
-    for (int i = i0 + tid; i < i1; i += BF_THREADS) {
-        const uint32_t info = ldg<uint32_t>(c.slot + i);
-        const float wv = ldg<float>(c.w + i);
-        const int t = i / SLOTS;
-        uint32_t p = 0xFFFFFFFFu;
-        if (info == PF_SLOT_HOLE) {
-            hole(t);
-        } else if (info != 0xFFFFFFFFu) {
-            if (info & PF_SLOT_NO_SHARED) hole(t);
-            const uint32_t e = info >> PF_SLOT_RANK_BITS, k = (info >> PF_SLOT_COPY_SHIFT) & (PF_CNT_COPIES - 1u);
-            p = S.rg[e] + (e < (uint32_t)E1 - 1u ? cb[k * E1 + e] : 0u) + (info & (PF_SLOT_NO_SHARED - 1u));
-            b.sorted_tok[p] = (uint16_t)t;
-            b.sorted_w[p] = wv;
-        }
-        b.pos[i] = p;
+    for (int i = i0 + tid; i < i1; i += BF_THREADS)
+        place_slot(b, S, cb, i, ldg<uint32_t>(c.slot + i), ldg<float>(c.w + i));
+}
+
+// Both steps of the fill in one launch for few tokens: workgroup 0 routes or reads the tokens,
+// counts and ranks them in LDS (no global counters), scans and places; the others prep as in
+// k_pf_place.  It saves a launch and the counters' way through L2, and puts the tokens on one CU: a
+// wave routes one (16 waves; the waves already share the SIMDs, so a second one each takes as long
+// again) or reads two (three still gain at M = 48; a call of 40 tokens with given ids keeps its two
+// timed launches, which the timing hook's callers count).  Measured, one layer in a graph, two launches -> one (us):
+//                   routed: M = 9        16        32     given: M = 9        21        48        64
+//     E = 256 uniform  49.8 -> 48.0  67.7 -> 66.8  93.6 -> 96.0  48.2 -> 45.7  69.1 -> 66.5  95.1 -> 93.5  110 -> 112
+//     E = 64 Zipf      30.0 -> 28.3  30.6 -> 29.3  43.7 -> 45.0  28.5 -> 26.2  37.6 -> 35.7  45.8 -> 44.1  49.7 -> 50.3
+template <bool ROUTE>
+constexpr int pf_fill_one_max_m() { return BF_THREADS / 64 * (ROUTE ? 1 : 2); }
+
+template <int H, bool ROUTE>
+__global__ __launch_bounds__(BF_THREADS) void k_pf_fill_one(BucketArgs b, PfCountArgs c, PrefillArgs a) {
+    const int tid = (int)threadIdx.x, wv = tid >> 6, lane = tid & 63;
+    if (blockIdx.x > 0) {
+        const int t = ((int)blockIdx.x - 1) * PF_PREP_TOKENS + wv;
+        if (wv < PF_PREP_TOKENS && t < a.M) prep_token<H>(a, t, lane); // whole waves
+        return;
     }
+    extern __shared__ uint32_t smem[];
+    constexpr int NW = BF_THREADS / 64, MMAX = pf_fill_one_max_m<ROUTE>(), PER = MMAX / NW;
+    __shared__ uint32_t info[SLOTS * MMAX];
+    __shared__ float w[SLOTS * MMAX];
+    const int E1 = b.E1;
+    const BucketScan S = bucket_scan_lds(smem, E1);
+    for (int e = tid; e < E1; e += BF_THREADS) S.tot[e] = e == E1 - 1 ? (uint32_t)b.M : 0u; // counted below
+    __syncthreads();
+    int id[PER];
+    float wt[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int t = wv + NW * u; // whole waves
+        id[u] = 0, wt[u] = 0.0f;
+        if (t >= b.M) continue;
+        if constexpr (ROUTE) {
+            route_wave<4>(c.logits + (size_t)t * c.E, c.E, c.renorm, lane, id[u], wt[u]);
+        } else if (lane < SLOTS) {
+            id[u] = (int)c.ids[t * SLOTS + lane];
+            wt[u] = c.w[t * SLOTS + lane];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int t = wv + NW * u;
+        if (t >= b.M) continue;
+        const CountedSlot k = count_token<ROUTE>(c, t, true, lane, id[u], wt[u], S.tot);
+        if (lane < SLOTS) {
+            info[t * SLOTS + lane] = slot_info(k, c.E, t, lane, 0u, 0u);
+            w[t * SLOTS + lane] = wt[u];
+        }
+    }
+    __syncthreads();
+    bucket_lists(b, S, true);
+    for (int i = tid; i < SLOTS * b.M; i += BF_THREADS) place_slot(b, S, nullptr, i, info[i], w[i]);
 }
 
 // ---------------------------------------------------------------- shared pipeline pieces
@@ -970,18 +1040,24 @@ template <int H, int I, bool TILED>
 static hipError_t launch_prefill_t(const BucketArgs &b, const PfCountArgs &c, const PrefillArgs &a, hipStream_t st,
                                    KernelTimer *T) {
     // the chain's own fill: count (routing first with logits), then place + prep
-    {
+    const int nprep = (a.M + PF_PREP_TOKENS - 1) / PF_PREP_TOKENS;
+    const size_t scan_lds = 5 * (size_t)(b.E1 + 1) * 4;
+    if (a.M <= (c.logits ? pf_fill_one_max_m<true>() : pf_fill_one_max_m<false>())) {
         TimedLaunch tl(T, c.logits ? MOE_K_ROUTER_TOPK : MOE_K_BUCKET_FILL, st);
-        const dim3 grid((unsigned)((c.M + PF_COUNT_TOKENS - 1) / PF_COUNT_TOKENS));
-        if (c.logits) hipLaunchKernelGGL(k_pf_count<true>, grid, dim3(64 * PF_COUNT_TOKENS), 0, st, c);
-        else hipLaunchKernelGGL(k_pf_count<false>, grid, dim3(64 * PF_COUNT_TOKENS), 0, st, c);
-    }
-    {
+        const dim3 grid((unsigned)(1 + nprep));
+        if (c.logits) hipLaunchKernelGGL((k_pf_fill_one<H, true>), grid, dim3(BF_THREADS), scan_lds, st, b, c, a);
+        else hipLaunchKernelGGL((k_pf_fill_one<H, false>), grid, dim3(BF_THREADS), scan_lds, st, b, c, a);
+    } else {
+        {
+            TimedLaunch tl(T, c.logits ? MOE_K_ROUTER_TOPK : MOE_K_BUCKET_FILL, st);
+            const dim3 grid((unsigned)((c.M + PF_COUNT_TOKENS - 1) / PF_COUNT_TOKENS));
+            if (c.logits) hipLaunchKernelGGL(k_pf_count<true>, grid, dim3(64 * PF_COUNT_TOKENS), 0, st, c);
+            else hipLaunchKernelGGL(k_pf_count<false>, grid, dim3(64 * PF_COUNT_TOKENS), 0, st, c);
+        }
         TimedLaunch tl(T, MOE_K_BUCKET_FILL, st);
         const int nplace = (SLOTS * b.M + PF_PLACE_SLOTS - 1) / PF_PLACE_SLOTS;
-        const int nprep = (a.M + PF_PREP_TOKENS - 1) / PF_PREP_TOKENS;
         hipLaunchKernelGGL((k_pf_place<H>), dim3((unsigned)(nplace + nprep)), dim3(BF_THREADS),
-                           (5 * (size_t)(b.E1 + 1) + (size_t)PF_CNT_COPIES * b.E1) * 4, st, b, c, a);
+                           scan_lds + (size_t)PF_CNT_COPIES * b.E1 * 4, st, b, c, a);
     }
     // one launch over the tile list (full and big remainder tiles, then small remainders, then
     // empty entries, which exit at once)

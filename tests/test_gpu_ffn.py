@@ -326,6 +326,49 @@ def test_prefill_nine_routed_slots(gpu, orc, M):
     ctx.close()
 
 
+@pytest.mark.parametrize("n_experts", [16, 64, E])
+def test_prefill_fill_edges(gpu, orc, n_experts):
+    """The bucket fill in one launch (routed tokens up to 16, given ids up to 32) and in two: the same
+    tokens give the same y, ids and weights bit for bit on both sides of the rule, also with repeated,
+    out-of-range and nine routed ids, and the routed call equals routing and the given-ids call."""
+    import torch
+    MX = 52
+    ctx = gpu.Context(512, 256, n_experts, 1, MX, gpu.W_REF)
+    layer = Layer(gpu, orc, 31, 512, 256, n_experts)
+    ctx.bind_packed(0, layer.dev)
+    x = gpu.gen_normal(MX * 512, 4001).view(MX, 512)
+    logits = gpu.gen_logits(MX, n_experts, 4002)
+    ids, w = ctx.router_topk(logits)
+    ids_h, w_h = ids.cpu().numpy().copy(), w.cpu().numpy()
+    y_ref = ctx.ffn(0, x, ids, w).clone()          # 52 tokens: two launches
+    for M in (9, 15, 16, 17, 31, 32, 33, 48):
+        y, i1, w1 = ctx.ffn_route(0, x[:M], logits[:M])
+        torch.cuda.synchronize()
+        assert torch.equal(i1, ids[:M]) and torch.equal(w1, w[:M]) and torch.equal(y, y_ref[:M]), M
+        y = ctx.ffn(0, x[:M], ids[:M].contiguous(), w[:M].contiguous())
+        torch.cuda.synchronize()
+        assert torch.equal(y, y_ref[:M]), M
+    assert ctx.device_flags() == 0
+    ids_h[1, 4] = ids_h[1, 1]            # a repeat
+    ids_h[2, 6] = n_experts + 5          # out of range
+    ids_h[3, :] = n_experts + 7          # no valid slot
+    ids_h[4, 2] = n_experts              # the shared expert in a routed slot: slot 8 repeats it
+    ids_h[5, 8] = next(e for e in range(n_experts) if e not in ids_h[5])  # nine routed experts
+    ids_h[6, 8] = ids_h[6, 0]            # no shared slot, slot 8 dropped
+    bad = torch.from_numpy(ids_h).cuda()
+    both = gpu.DEVFLAG_BAD_ID | gpu.DEVFLAG_DUP_ID
+    y_ref = ctx.ffn(0, x, bad, w).clone()
+    torch.cuda.synchronize()
+    assert ctx.device_flags() == both
+    check_errs(y_ref.cpu().numpy(), orc.moe_ffn(layer.host(), x.cpu().numpy(), ids_h, w_h, 1.0 / 9), False)
+    for M in (9, 16, 17, 31, 32, 33):
+        y = ctx.ffn(0, x[:M], bad[:M].contiguous(), w[:M].contiguous())
+        torch.cuda.synchronize()
+        assert ctx.device_flags() == both
+        assert torch.equal(y, y_ref[:M]), M
+    ctx.close()
+
+
 def test_prefill_dropped_slots_skip_nonfinite_row0(gpu, orc, full):
     """Prefill (M = 16): token 0 routes to expert 0 in slot 0, so its partial output is
     expert-sorted row 0, and its activations are +inf (that row is non-finite).  Token 1 names
