@@ -3,13 +3,13 @@
 // Replaces the reference's bucketed prefill dispatches (src/inference.rs:683-732): per
 // non-empty bucket a tiled w1_w3_fused GEMM into an f16 scratch and a w2_scatter GEMM
 // whose epilogue read-modify-writes the f16 hidden state (shaders/w1_w3_fused.comp,
-// shaders/w2_scatter.comp).  Here, after the chain's bucket fill (k_pf_count, k_pf_place,
-// below) has produced expert-sorted slots and a list of tiles (up to PF_BM slots of one
+// shaders/w2_scatter.comp).  Here, after the chain's bucket fill (k_pf_count, k_pf_place, or
+// k_pf_fill_one, below) has produced expert-sorted slots and a list of tiles (up to PF_BM slots of one
 // expert):
 //   prep:    per token, x (RMSNorm fused when asked) times a power of two s_t that puts
 //            max|x| in [2^14, 2^15), stored as f16 with K permuted inside 32-blocks (the
 //            order the weight nibbles arrive in, see below); 1/s_t kept per token -- run in
-//            the same launch as the slot placement (k_pf_place), which does not need it;
+//            the same launch as the slot placement, which does not need it;
 //   gate_up: per (tile, 64 gate/up column pairs; 128 when M > 512) a workgroup of 8 waves,
 //            two per CU; the tile's token rows (gathered -- the reference's kernel skipped
 //            this gather) are resident in LDS one 64 KB chunk of K at a time and shared by the
@@ -418,8 +418,9 @@ __device__ __forceinline__ const T *uniform_ptr(const T *p) {
 // TILED: from the tiled copy (k_repack_tiled), where the 1 KB of a load is contiguous and in lane
 // order; else from the split copy (k_repack_split; a context without the tiled one: moe_create), where
 // a row's bytes are together, so neighbouring lanes read rows 128 SBR bytes apart and the address
-// unit takes them one by one.  Measured, one layer, split -> tiled (us): M = 21 83.0 -> 77.7,
-// M = 512 (Zipf) 116 -> 109, M = 4096 467 -> 448.
+// unit takes them one by one.  Measured, one layer, split -> tiled (us), E = 256 uniform / E = 128 Zipf:
+// M = 21 83 -> 77 / 46.0 -> 43.5, M = 100 131 -> 120 / 57.3 -> 53.0, M = 512 156 -> 141 / 108 -> 101,
+// M = 4096 458 -> 434 / 424 -> 404.
 template <bool TILED>
 struct WRows {
     const uint8_t *q; // qs of the 16-row group: TILED, stage c at 1024 c; else its first row's

@@ -174,13 +174,13 @@ __global__ __launch_bounds__(64 * RG_WAVES) void k_router_gemv(RouterGemvArgs a)
 // tokens' RMSNorm factors come from the same x registers.
 // K inside a stage: the order is free as long as both operands agree.  Lane (g, i) takes K =
 // 16 q + 4 g + j of row i (q < 2, j < 4), so the four lanes of a row read 64 consecutive bytes of
-// x per load (with 32 consecutive K per lane pair the loads, one cache line per lane, took as long
-// as the MFMAs), and one IQ4_XS qs dword has the lane's 8 weights: low nibbles q = 0, high q = 1.
+// x per load, and one IQ4_XS qs dword has the lane's 8 weights: low nibbles q = 0, high q = 1.
 // Rounding: an MFMA chain covers one stage (32 K); the chains are added in f32 per wave and the
 // waves' sums and the RMSNorm factor taken in f64.  Relative 2-norm against f64 (E = 256): 1.2e-7
 // (1.34e-7 in the 64 x 64 form) for every gate type, the one-row form 1.34e-7 (IQ4_XS 2.6e-7).
 // f16 gate, M = 4096: 947 -> 48 us; the f32 matrix cores alone need 31 us at their measured
-// 139 TFLOP/s.
+// 139 TFLOP/s.  Bound by one wave's chain of f32 MFMAs and conversions per SIMD: with both operands staged
+// in LDS instead the 64 x 64 form takes 44.8 us against 46.6, and its error is larger (1.54e-7).
 template <int WT>
 struct RmW; // a lane's 8 weights of one stage as loaded; off: byte offset of the lane's first one
 template <>
@@ -374,8 +374,8 @@ static int rm_tiles(const RouterGemvArgs &a) {
 //     16 x 16           8.0    9.2    9.2    9.4  17.3   33.2   65.1    127
 //     32 x 32          13.8   15.2   18.2   18.3  18.5   19.1   35.5   68.1
 //     64 x 64          41.2   41.5   43.3   43.7  43.7   43.4   43.9   45.8
-// Every 16 x 16 or 64 x 64 workgroup has a CU to itself and takes the same time whatever M is:
-// its rows lie 8 KB apart, so the rows of a load share an L2 channel.
+// A workgroup of the 64 x 64 form takes the same ~41 us whatever M is (its waves' f32 MFMAs over all of
+// K), so the smaller tiles win until they need a second round on the CUs.
 template <int H, int WT>
 static void launch_router_gemv_w(const RouterGemvArgs &a, hipStream_t st) {
     // a wave's tokens past M repeat the last one: at small M fewer tokens per wave

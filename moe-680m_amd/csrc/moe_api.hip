@@ -195,7 +195,7 @@ moe_status moe_create(int device, const moe_config *cfg, moe_ctx **out) {
                         hipGetErrorString(he));
         }
         // the tiled copy only where half of the device's memory stays free beside it: without it
-        // the prefill GEMMs read the split copy, 4 to 8 % more slowly
+        // the prefill GEMMs read the split copy, 5 to 11 % more slowly (wstage_load)
         size_t mfree = 0, mtotal = 0;
         if (cfg->m_max > MOE_DECODE_MAX_M && hipMemGetInfo(&mfree, &mtotal) == hipSuccess &&
             mfree >= sbytes + mtotal / 2 && hipMalloc((void **)&c->tpk, sbytes) != hipSuccess)

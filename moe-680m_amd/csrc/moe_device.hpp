@@ -9,8 +9,8 @@
 // It replaces the reference's 36-byte block decoder (shaders/common.glsl:61-86), which
 // re-read d and both bit planes per weight through 8-bit word loads.  Here a lane owns one
 // sub-block: the 8-byte header and the 16 qs bytes arrive as one 64-bit and one 128-bit
-// load, the codebook lookup is three v_perm_b32 per four weights, and the scale is applied
-// once per sub-block.
+// load, the codebook lookup is two v_perm_b32 and an XOR per four weights (the decode stack:
+// three v_perm_b32), and the scale is applied once per sub-block.
 #pragma once
 
 #include <hip/hip_runtime.h>
