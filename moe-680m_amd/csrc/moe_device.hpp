@@ -88,8 +88,9 @@ constexpr XorTable xor_table(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3)
 template <uint32_t T0, uint32_t T1, uint32_t T2, uint32_t T3>
 __device__ __forceinline__ uint32_t lookup16(uint32_t idx) {
     constexpr XorTable X = xor_table(T0, T1, T2, T3);
-    uint32_t flip; // in asm: the compiler makes (q & m) ^ 8 a v_bitop3 (4.4 cycles) instead of this v_xor (2.4)
-    asm("v_xor_b32 %0, %1, %2" : "=v"(flip) : "s"(0x08080808u), "v"(idx));
+    // Plain C++, not asm: the compiler puts the wait states that an MFMA's registers need in front
+    // of its own instructions only (and Makefile's NO_BITOP3 keeps it from making a v_bitop3 of this).
+    const uint32_t flip = idx ^ 0x08080808u;
     return __builtin_amdgcn_perm(X.t[1], X.t[0], idx) ^ __builtin_amdgcn_perm(X.t[3], X.t[2], flip);
 }
 
