@@ -85,14 +85,26 @@ typedef struct {
 
 /* Create a context on HIP device `device`: validates the shape, allocates every
  * workspace for m_max tokens and the device copies of the weights that moe_bind_layer
- * fills (nothing is allocated later): n_layers x (E+1) x 3 matrices in the library's split
- * layout, which the decode kernels read, and -- with m_max > MOE_DECODE_MAX_M, and only where
- * half of the device's memory stays free beside it -- the same in the tiled layout of the
- * prefill GEMMs (which otherwise read the split one; the results are the same bit for bit).
+ * fills (nothing is allocated later): moe_create_with and MOE_COPIES_AUTO.
  * Replaces the MoE slice of InferenceEngine::new (src/inference.rs:85-126) and the
  * scratch / routing regions of ArenaLayout::compute (src/memory.rs:32-96). */
 moe_status moe_create(int device, const moe_config *cfg, moe_ctx **out);
 moe_status moe_destroy(moe_ctx *ctx);
+
+/* The device copies of the weights that a context keeps, each n_layers x (E+1) x 3 matrices:
+ * the split layout, which the decode kernels read and the prefill GEMMs can, and the tiled one,
+ * from which the prefill GEMMs (M > MOE_DECODE_MAX_M) run some percent faster; the results are
+ * the same bit for bit. */
+enum {
+    MOE_COPIES_AUTO = 0,  /* split; tiled too with m_max > MOE_DECODE_MAX_M, where it takes at most an
+                             eighth of the device's memory and half of that memory stays free beside it */
+    MOE_COPIES_SPLIT = 1, /* split only: half the memory */
+    MOE_COPIES_BOTH = 2   /* both, or MOE_ENOMEM: the same speed whatever else is allocated */
+};
+/* moe_create with that choice made by the caller. */
+moe_status moe_create_with(int device, const moe_config *cfg, int copies, moe_ctx **out);
+/* Device bytes of a context's two copies (*tiled 0: it has none).  No reference counterpart. */
+moe_status moe_weight_bytes(moe_ctx *ctx, size_t *split, size_t *tiled);
 
 /* Copy one layer's weights (device pointers, read only during this call) into the context's
  * layouts (same bytes, qs and headers of each super-block apart).  Synchronises the

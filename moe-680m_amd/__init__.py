@@ -37,6 +37,7 @@ MOE_OK, MOE_EINVAL, MOE_ENOMEM, MOE_EHIP, MOE_EUNSUPPORTED, MOE_EDEVICE = range(
 STATUS_NAMES = {0: "MOE_OK", 1: "MOE_EINVAL", 2: "MOE_ENOMEM", 3: "MOE_EHIP",
                 4: "MOE_EUNSUPPORTED", 5: "MOE_EDEVICE"}
 W_REF, W_RENORM = 0, 1
+COPIES_AUTO, COPIES_SPLIT, COPIES_BOTH = 0, 1, 2
 FFN_ACCUMULATE, FFN_RMSNORM, STACK_ROUTE_GEMV = 1, 2, 4
 DEVFLAG_BAD_ID, DEVFLAG_DUP_ID, DEVFLAG_TIMEOUT = 1, 2, 4
 # Router gate matrix element types (GGML type ids, include/moe_ffn.h MOE_WG_*).
@@ -44,7 +45,7 @@ WG_F32, WG_F16, WG_IQ4_XS = 0, 1, 23
 
 # Every symbol include/moe_ffn.h declares (checked by the CPU test suite).
 EXPORTS = (
-    "moe_create", "moe_destroy", "moe_bind_layer", "moe_bind_router", "moe_router_topk", "moe_router_gemv_topk",
+    "moe_create", "moe_create_with", "moe_destroy", "moe_weight_bytes", "moe_bind_layer", "moe_bind_router", "moe_router_topk", "moe_router_gemv_topk",
     "moe_router_gemv_topk_typed", "moe_bucket_fill",
     "moe_ffn", "moe_ffn_route", "moe_ffn_noalloc", "moe_decode_stack", "moe_dequant_iq4xs", "moe_device_flags",
     "moe_device_flags_async", "moe_stack_spin_limit", "moe_stack_trace", "moe_last_error",
@@ -89,7 +90,9 @@ def lib():
     vp, i, u64, sz = ctypes.c_void_p, ctypes.c_int, ctypes.c_uint64, ctypes.c_size_t
     sigs = {
         "moe_create": [i, ctypes.POINTER(_Config), ctypes.POINTER(vp)],
+        "moe_create_with": [i, ctypes.POINTER(_Config), i, ctypes.POINTER(vp)],
         "moe_destroy": [vp],
+        "moe_weight_bytes": [vp, ctypes.POINTER(sz), ctypes.POINTER(sz)],
         "moe_bind_layer": [vp, i, ctypes.POINTER(_LayerWeights)],
         "moe_router_topk": [vp, vp, i, vp, vp, vp],
         "moe_router_gemv_topk": [vp, vp, vp, i, i, vp, vp, vp, vp],
@@ -158,15 +161,17 @@ def layer_bytes(hidden, inter, n_experts):
 
 
 class Context:
-    """One moe_ctx: shapes, per-layer weight tables and all workspaces."""
+    """One moe_ctx: shapes, per-layer weight tables and all workspaces.  copies: the device
+    copies of the weights it keeps -- COPIES_AUTO, COPIES_SPLIT (half the memory) or COPIES_BOTH
+    (include/moe_ffn.h)."""
 
     def __init__(self, hidden=2048, inter=512, n_experts=256, n_layers=1, m_max=512,
-                 wmode=W_REF, device=0):
+                 wmode=W_REF, device=0, copies=COPIES_AUTO):
         self.hidden, self.inter, self.n_experts = hidden, inter, n_experts
         self.n_layers, self.m_max, self.wmode, self.device = n_layers, m_max, wmode, device
         cfg = _Config(hidden, inter, n_experts, n_layers, m_max, wmode)
         h = ctypes.c_void_p()
-        _check(lib().moe_create(device, ctypes.byref(cfg), ctypes.byref(h)))
+        _check(lib().moe_create_with(device, ctypes.byref(cfg), copies, ctypes.byref(h)))
         self._h = h
 
     @property
@@ -183,6 +188,12 @@ class Context:
             self.close()
         except Exception:
             pass
+
+    def weight_bytes(self):
+        """(split, tiled): device bytes of the two weight copies, tiled 0 if there is none."""
+        split, tiled = ctypes.c_size_t(), ctypes.c_size_t()
+        _check(lib().moe_weight_bytes(self._h, ctypes.byref(split), ctypes.byref(tiled)))
+        return split.value, tiled.value
 
     def bind_layer(self, layer, w1, w3, w2, w1_stride, w3_stride, w2_stride,
                    shared_w1, shared_w3, shared_w2):

@@ -24,8 +24,8 @@ struct moe_ctx {
     std::vector<LayerPtrs> tlayers; // ... and its tiled copy, when there is one
     std::vector<char> bound;
     uint8_t *spk = nullptr;         // [n_layers][E+1][W1|W3|W2] split layout (decode kernels)
-    uint8_t *tpk = nullptr;         // the same matrices tiled (prefill GEMMs): m_max > MOE_DECODE_MAX_M and
-                                    // ample device memory, else null and the GEMMs read spk
+    uint8_t *tpk = nullptr;         // the same matrices tiled (prefill GEMMs), or null: the GEMMs read spk
+    size_t copy_bytes = 0;          // of each copy
     void *arena = nullptr; // one device allocation, carved below
     size_t arena_bytes = 0;
     uint32_t *flags = nullptr;   // [0] sticky device flags, [1] the decode stack's abort word
@@ -113,8 +113,14 @@ extern "C" {
 const char *moe_last_error(void) { return g_err.c_str(); }
 
 moe_status moe_create(int device, const moe_config *cfg, moe_ctx **out) {
+    return moe_create_with(device, cfg, MOE_COPIES_AUTO, out);
+}
+
+moe_status moe_create_with(int device, const moe_config *cfg, int copies, moe_ctx **out) {
     if (!cfg || !out) return fail(MOE_EINVAL, "moe_create: null argument");
     *out = nullptr;
+    if (copies != MOE_COPIES_AUTO && copies != MOE_COPIES_SPLIT && copies != MOE_COPIES_BOTH)
+        return fail(MOE_EINVAL, "moe_create_with: unknown copies %d", copies);
     const int H = cfg->hidden, I = cfg->inter, E = cfg->n_experts;
     if (!shape_compiled(H, I))
         return fail(MOE_EUNSUPPORTED, "moe_create: hidden=%d inter=%d not compiled (2048x512, 512x256)", H, I);
@@ -194,13 +200,22 @@ moe_status moe_create(int device, const moe_config *cfg, moe_ctx **out) {
             return fail(MOE_ENOMEM, "moe_create: hipMalloc(%zu) for the weight copies: %s", sbytes,
                         hipGetErrorString(he));
         }
-        // the tiled copy only where half of the device's memory stays free beside it: without it
-        // the prefill GEMMs read the split copy, 5 to 11 % more slowly (wstage_load)
-        size_t mfree = 0, mtotal = 0;
-        if (cfg->m_max > MOE_DECODE_MAX_M && hipMemGetInfo(&mfree, &mtotal) == hipSuccess &&
-            mfree >= sbytes + mtotal / 2 && hipMalloc((void **)&c->tpk, sbytes) != hipSuccess)
-            c->tpk = nullptr;
-        (void)hipGetLastError();
+        c->copy_bytes = sbytes;
+        bool tiled = copies == MOE_COPIES_BOTH;
+        if (copies == MOE_COPIES_AUTO && cfg->m_max > MOE_DECODE_MAX_M) {
+            size_t mfree = 0, mtotal = 0;
+            he = hipMemGetInfo(&mfree, &mtotal);
+            tiled = he == hipSuccess && sbytes <= mtotal / 8 && mfree >= sbytes + mtotal / 2;
+        }
+        if (tiled && (he = hipMalloc((void **)&c->tpk, sbytes)) != hipSuccess) c->tpk = nullptr;
+        if (he != hipSuccess) (void)hipGetLastError(); // reported here, or AUTO without the tiled copy
+        if (copies == MOE_COPIES_BOTH && !c->tpk) {
+            (void)hipFree(c->spk);
+            (void)hipFree(c->arena);
+            delete c;
+            return fail(MOE_ENOMEM, "moe_create: hipMalloc(%zu) for the tiled weight copy: %s", sbytes,
+                        hipGetErrorString(he));
+        }
     }
     c->xtag_words = STK_CTL_WORDS + 2 * (size_t)cfg->n_layers * stack_layer_words(H, I);
     he = hipMemset(c->flags, 0, 256);
@@ -245,6 +260,13 @@ moe_status moe_destroy(moe_ctx *ctx) {
     hipError_t he = hipFree(ctx->arena);
     delete ctx;
     if (he != hipSuccess) return hip_fail(he, "moe_destroy: hipFree");
+    return ok();
+}
+
+moe_status moe_weight_bytes(moe_ctx *ctx, size_t *split, size_t *tiled) {
+    if (!ctx || !split || !tiled) return fail(MOE_EINVAL, "moe_weight_bytes: null argument");
+    *split = ctx->copy_bytes;
+    *tiled = ctx->tpk ? ctx->copy_bytes : 0;
     return ok();
 }
 

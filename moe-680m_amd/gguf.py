@@ -289,18 +289,19 @@ def load_layers(ctx, path, layers=None, file_layers=None, device="cuda"):
     return routers
 
 
-def open_context(path, m_max, wmode=None, device=0):
+def open_context(path, m_max, wmode=None, device=0, copies=0):
     """A Context sized from the file's metadata (model_config) with every layer bound, and the
     routers load_layers returns: the loader role of the reference's InferenceEngine::new for
     this path (src/inference.rs:85-126 with src/gguf.rs:147-212 and src/memory.rs:227-291).
-    The file must route 8 experts per token (expert_used_count), as this path does."""
+    The file must route 8 experts per token (expert_used_count), as this path does.  copies:
+    as Context's (0 = COPIES_AUTO)."""
     from . import W_RENORM, Context, TOPK
     with GGUFFile(path) as g:
         cfg = model_config(g)
     if cfg["n_experts_used"] != TOPK:
         raise GGUFError(f"expert_used_count {cfg['n_experts_used']}: this path routes {TOPK} experts per token")
     ctx = Context(cfg["hidden"], cfg["inter"], cfg["n_experts"], cfg["n_layers"], m_max,
-                  W_RENORM if wmode is None else wmode, device=device)
+                  W_RENORM if wmode is None else wmode, device=device, copies=copies)
     try:
         routers = load_layers(ctx, path, device=f"cuda:{device}")
     except Exception:

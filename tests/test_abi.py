@@ -47,6 +47,8 @@ def test_host_validation_without_gpu(pkg):
     assert L.moe_dequant_iq4xs(None, 1, None, None) == pkg.MOE_EINVAL
     assert L.moe_bind_layer(None, 0, None) == pkg.MOE_EINVAL
     assert L.moe_create(0, None, ctypes.byref(vp())) == pkg.MOE_EINVAL
+    assert L.moe_create_with(0, None, 0, ctypes.byref(vp())) == pkg.MOE_EINVAL
+    assert L.moe_weight_bytes(None, None, None) == pkg.MOE_EINVAL
     # shape that is not compiled -> MOE_EUNSUPPORTED before any HIP call
     cfg = pkg._Config(4096, 512, 256, 1, 16, 0)
     h = vp()

@@ -163,25 +163,58 @@ def test_prefill_tile_heights(gpu, orc, full, M, n):
     check_errs(y.cpu().numpy()[t], ref, False)
 
 
-def test_prefill_from_split_copy(gpu, full):
-    """A context whose weights leave too little device memory free for the tiled copy runs the
-    prefill GEMMs from the split copy: the same y bit for bit, every tile height and both item
-    widths (the same weights, bound to both contexts)."""
+@pytest.mark.parametrize("hidden,inter,nexp", [(H, I, E), (512, 256, 16)])
+def test_prefill_from_split_copy(gpu, orc, hidden, inter, nexp):
+    """A context without the tiled copy runs the prefill GEMMs from the split copy: the same y bit
+    for bit, every tile height, both item widths and both compiled shapes (the same weights, bound
+    to both contexts, whose copies are the ones asked for)."""
     import torch
-    ctx, layer = full
+    layer = Layer(gpu, orc, 41, hidden, inter, nexp)
+    both = gpu.Context(hidden, inter, nexp, 1, 1100, gpu.W_REF, copies=gpu.COPIES_BOTH)
+    split = gpu.Context(hidden, inter, nexp, 1, 1100, gpu.W_REF, copies=gpu.COPIES_SPLIT)
+    nbytes = gpu.layer_bytes(hidden, inter, nexp)
+    assert both.weight_bytes() == (nbytes, nbytes)
+    assert split.weight_bytes() == (nbytes, 0)
+    for c in (both, split):
+        c.bind_packed(0, layer.dev)
+    for M in (9, 40, 512, 513, 1100):
+        x = gpu.gen_normal(M * hidden, 3500 + M).view(M, hidden)
+        ids, w = both.router_topk(gpu.gen_logits(M, nexp, 3501 + M, kind=1, param=1.1))
+        y0, y1 = both.ffn(0, x, ids, w), split.ffn(0, x, ids, w)
+        torch.cuda.synchronize()
+        assert torch.equal(y0, y1), M
+        t = np.r_[0:4, M - 4:M]
+        ref = orc.moe_ffn(layer.host(), x.cpu().numpy()[t], ids.cpu().numpy()[t], w.cpu().numpy()[t], 1.0 / 9)
+        check_errs(y1.cpu().numpy()[t], ref, False)
+    both.close()
+    split.close()
+
+
+def test_weight_copies(gpu):
+    """The copies a context makes on its own, what each takes, and what a caller can ask for: by
+    default the tiled copy where prefill calls can come, and never above an eighth of the device."""
+    import torch
+    nbytes = gpu.layer_bytes(512, 256, 16)
+
+    def copies(n_layers, m_max, **kw):
+        c = gpu.Context(512, 256, 16, n_layers, m_max, gpu.W_REF, **kw)
+        got = c.weight_bytes()
+        c.close()
+        return got
+
+    assert copies(3, 8) == (3 * nbytes, 0)
+    assert copies(3, 9) == (3 * nbytes, 3 * nbytes)
+    assert copies(3, 9, copies=gpu.COPIES_SPLIT) == (3 * nbytes, 0)
+    assert copies(3, 8, copies=gpu.COPIES_BOTH) == (3 * nbytes, 3 * nbytes)
     total = torch.cuda.mem_get_info()[1]
-    n_layers = int(0.35 * total) // gpu.layer_bytes(H, I, E)
-    big = gpu.Context(H, I, E, n_layers, 1100, ctx.wmode)
-    try:
-        big.bind_packed(n_layers - 1, layer.dev)
-        for M in (9, 40, 512, 513, 1100):
-            x = gpu.gen_normal(M * H, 3500 + M).view(M, H)
-            ids, w = ctx.router_topk(gpu.gen_logits(M, E, 3501 + M, kind=1, param=1.1))
-            y0, y1 = ctx.ffn(0, x, ids, w), big.ffn(n_layers - 1, x, ids, w)
-            torch.cuda.synchronize()
-            assert torch.equal(y0, y1), M
-    finally:
-        big.close()
+    n = total // 8 // gpu.layer_bytes(H, I, E) + 1
+    c = gpu.Context(H, I, E, n, 16, gpu.W_REF)
+    assert c.weight_bytes() == (n * gpu.layer_bytes(H, I, E), 0)
+    c.close()
+    for bad in (-1, 3):
+        with pytest.raises(gpu.MoeError) as e:
+            gpu.Context(512, 256, 16, 1, 16, gpu.W_REF, copies=bad)
+        assert e.value.status == gpu.MOE_EINVAL
 
 
 @pytest.fixture(scope="module")
