@@ -651,9 +651,9 @@ __device__ __forceinline__ void by_mtiles(int nrows, F f) {
 // XCD w % 8, so tile 8 (k / ITEMS) + w % 8, item k % ITEMS (k = w / 8) puts every item of a
 // tile on one XCD -- the tile's token rows (gate/up) or h rows (down) come from HBM once and
 // are L2 hits for its other items -- and consecutive tiles on consecutive XCDs, in dispatch
-// order.  Used for the wide items of large M (measured, M = 4096: gate/up 310 -> 292 us, down
-// 189 -> 176 us); at M <= 512 the rows of all the tiles stay in the memory-side cache anyway
-// and one tile's items spread over the eight XCDs run faster (M = 512: 124 against 132 us).
+// order.  Used for the wide items (measured when they came in, M = 4096: gate/up 310 -> 292 us, down
+// 189 -> 176 us); with the 64-column items the rows of all the tiles stay in the memory-side cache
+// anyway and one tile's items spread over the eight XCDs run faster (M = 512 then: 124 against 132 us).
 template <int ITEMS, bool GROUP>
 __device__ __forceinline__ void xcd_tile_item(int &tile, int &item) {
     if constexpr (GROUP) {

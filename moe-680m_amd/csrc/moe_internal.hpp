@@ -17,10 +17,20 @@ constexpr int PF_SMALL_MAX = 32; // remainders of at most this many slots are li
 // h columns per prefill gate/up work item, and per hmax block: 64 (two waves per 16 columns,
 // alternate K stages: half-length items, which fill the last round of workgroup slots better)
 // for M <= PF_SPLIT_MAX_M, else 128 (one wave per 16 columns: fewer items to stage A for, a tile's
-// items on one XCD).  Measured (H 2048, I 512, one layer, 64 / 128 columns, us): E = 256 uniform
-// M = 256 128.1 / 127.2, 512 154.5 / 142.3, 640 156.1 / 150.8; Zipf 256 82.4 / 80.4, 512 105.1 /
-// 108.4, 640 122.5 / 117.4; E = 128 uniform 150 80.7 / 82.5, 256 85.7 / 88.3, 512 107.9 / 104.9;
-// E = 64 256 72.0 / 74.0, 400 84.0 / 84.4, 512 92.6 / 88.9: above 512 every routing gains.
+// items on one XCD).  Time of the 128-column form over the 64-column one (H 2048, I 512, one routed
+// call, six layers in turn so that the weights come from memory; in brackets one layer again and again):
+//     M               128          192       256          320      384          448          512          640
+//     E = 256 uniform 0.98 (0.98)  (1.00)  0.99 (1.00)  (0.99)  0.99 (0.99)  0.98 (0.99)  0.98 (0.97)  0.99 (0.98)
+//     E = 256 Zipf    1.11 (1.12)  (1.00)  0.96 (0.97)  (0.96)  0.94 (0.94)  1.00 (1.01)  1.02 (0.99)  0.98 (0.97)
+//     E = 128 uniform 1.03 (1.03)  (1.02)  1.02 (1.05)  (1.02)  1.00 (1.01)  0.98 (0.97)  0.97 (0.97)  0.97 (0.96)
+//     E = 128 Zipf    1.14 (1.13)  (1.01)  0.97 (0.95)  (0.97)  0.95 (0.96)  1.00 (1.02)  1.03 (1.01)  0.98 (0.98)
+//     E = 64 uniform  1.13 (1.11)  (1.11)  1.05 (1.05)  (1.03)  1.01 (1.03)  1.01 (1.02)  0.96 (0.96)  0.97 (0.97)
+//     E = 64 Zipf     1.07 (1.06)  (1.10)  0.98 (0.97)  (0.98)  0.96 (0.97)  0.93 (0.96)  0.96 (0.98)  1.02 (1.01)
+//     mean            1.07 (1.07)  (1.04)  0.99 (1.00)  (0.99)  0.98 (0.98)  0.98 (0.99)  0.99 (0.98)  0.99 (0.98)
+// By how full the last round of workgroup slots is, either form is ahead at some loads from 256 to 640 by
+// up to 7 %; the 64-column form at most loads below, the 128-column form at all above.  The mean changes
+// sides at 256 already, but a line there takes from some loads what it gives to others (M = 512: E = 256
+// uniform 146 -> 142 us, Zipf 104.0 -> 106.3); from 513 on one load of the table loses (E = 64 Zipf at 640).
 constexpr int PF_NGU = 64;
 constexpr int PF_NGU_WIDE = 128;
 constexpr int PF_SPLIT_MAX_M = 512;

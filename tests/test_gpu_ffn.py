@@ -124,7 +124,7 @@ def test_config4_prefill_m4096_hot(gpu, orc, full):
 
 
 def test_prefill_m1024_every_token(gpu, orc, full):
-    """M in 769..1024: the wide (128-column) gate/up items with the keep-in-LDS bucket fill."""
+    """The wide (128-column) gate/up items at sizes between the two configurations'."""
     ctx, layer = full
     for M in (800, 1024):
         log(f"prefill M={M}, Zipf(1.1), all tokens checked")
