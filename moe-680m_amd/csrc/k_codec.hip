@@ -201,7 +201,8 @@ __global__ __launch_bounds__(256) void k_gen_logits(float *__restrict__ dst, int
 
 // ---------------------------------------------------------------- launchers
 // ---------------------------------------------------------------- split repack
-// One-time copy of a bound layer into the layout every kernel family reads.  Per matrix of nsb
+// One-time copy of a bound layer into the layout that the decode kernels read (and the prefill GEMMs
+// of a context without the tiled copy, below).  Per matrix of nsb
 // super-blocks (row-major: rows x super-blocks per row):
 //     [nsb x 128-byte qs] [nsb x 8-byte header (d, scales_h, scales_l)]
 // -- the bytes of the natural layout (136 per super-block) split in two, so that every

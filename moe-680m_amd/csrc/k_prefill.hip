@@ -418,9 +418,11 @@ __device__ __forceinline__ const T *uniform_ptr(const T *p) {
 // TILED: from the tiled copy (k_repack_tiled), where the 1 KB of a load is contiguous and in lane
 // order; else from the split copy (k_repack_split; a context without the tiled one: moe_create), where
 // a row's bytes are together, so neighbouring lanes read rows 128 SBR bytes apart and the address
-// unit takes them one by one.  Measured, one layer, split -> tiled (us), E = 256 uniform / E = 128 Zipf:
-// M = 21 83 -> 77 / 46.0 -> 43.5, M = 100 131 -> 120 / 57.3 -> 53.0, M = 512 156 -> 141 / 108 -> 101,
-// M = 4096 458 -> 434 / 424 -> 404.
+// unit takes them one by one.  Measured, one routed call, six layers in turn, split -> tiled (us), E = 256
+// uniform / E = 128 Zipf: M = 21 80.2 -> 72.4 / 44.8 -> 41.4, M = 100 129.0 -> 114.7 / 59.2 -> 55.0, M = 512 157.1
+// -> 142.4 / 109.3 -> 101.5, M = 4096 461.7 -> 443.8 / 416.2 -> 403.9; one layer again and again (its weights
+// partly cached) 73.0 -> 68.3 / 48.3 -> 45.4, 133.2 -> 118.5 / 59.3 -> 56.7, 160.6 -> 146.8 / 105.1 -> 100.6,
+// 465.5 -> 444.5 / 428.2 -> 410.1.
 template <bool TILED>
 struct WRows {
     const uint8_t *q; // qs of the 16-row group: TILED, stage c at 1024 c; else its first row's
@@ -631,7 +633,8 @@ __device__ __forceinline__ void gemm_resident_split(WStage<NR> (&ws)[RD], const 
 }
 
 // A tile holds up to PF_BM slots of one expert and runs as 1 to 4 M-tiles of 16 rows (one
-// instantiation each, picked per workgroup, so every inner loop is straight-line code).  Full
+// instantiation each, picked per workgroup, so every inner loop is straight-line code; with 4 for
+// 33 to 48 rows too, one layer, E = 256 uniform: M = 1000 173.8 -> 180.4 us, M = 1200 188.0 -> 197.8).  Full
 // PF_BM tiles come first in the list, remainders after: the long work items start first and
 // the short ones fill in.  64-row tiles, not 128: every wave reads each A fragment from LDS
 // once per pair of B fragments, so LDS traffic per K step grows with the tile height;
